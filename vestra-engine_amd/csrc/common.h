@@ -65,6 +65,10 @@ struct vk_linear {
   size_t out_features = 0;
   size_t k_pitch = 0;          // in_features rounded up to 16
   float* weight_nk = nullptr;  // [out, k_pitch], input dimension contiguous
+  // The rows as two f16 parts in the wide linear's fragment order, each row
+  // scaled by 2^weight_exp (split_weights), for in_features % 4 == 0.
+  void* weight_split = nullptr;
+  int* weight_exp = nullptr;   // [out], in weight_split's allocation
   // For a 3x14x14 patch filter (in_features 588) only: the same rows with
   // the input dimension reordered (c, ky, kx) -> (ky, kx, c), the order in
   // which an HWC image holds a patch.
@@ -168,6 +172,9 @@ void noalloc_setup(int device);
 // (c, ky, kx) -> (ky, kx, c) of an HWC image's patch, zero-padded to 592, on
 // the runtime's stream.  Any other linear: nothing.
 int prepare_patch_filter(vk_runtime* rt, vk_linear* lin);
+// Allocates and fills lin->weight_split and weight_exp from lin->weight_nk (whose writes have
+// finished); the default stream, waited for.  in_features % 4 != 0: nothing.
+int split_weights(vk_linear* lin);
 // Makes rt->work hold at least `floats` floats (at least 8 Mi once
 // allocated, doubling on growth).  Growth is refused during stream capture:
 // run the sequence once eagerly first.  The buffer it replaces is retired,
@@ -212,6 +219,8 @@ struct QkEpilogue {
 struct LinearArgs {
   const float* x;     // [M, K]
   const float* wnk;   // [N, Kp], K contiguous, zero beyond K
+  const void* wsplit; // its f16 parts (vk_linear::weight_split) and
+  const int* wexp;    // their rows' exponents, linear.hip only
   const float* bias;  // [N]
   const float* ls;    // [N] or null
   float* out;         // [M, N]
@@ -222,7 +231,7 @@ struct LinearArgs {
   float* v_out;
   int a_hnd;     // 1: x is head-major [K/64, M, 64] (the attention output)
   // split-K (linear.hip only): `splits` workgroups share each output tile,
-  // each over a contiguous run of 64-wide k chunks, writing raw sums to
+  // each over a contiguous run of 32-wide k stages, writing raw sums to
   // partial [splits, M, N]; a second pass adds them in split order and
   // applies the epilogue.
   int splits;
@@ -257,6 +266,10 @@ enum LinearEpilogue {
 // The wide-tile linear (128 x 128, 64 x 128 or 64 x 64 tiles, split-K for
 // few rows) for K % 4 == 0 and a 16-byte aligned x (linear.hip);
 // the head-major layouts of LinearArgs need it.
+constexpr int kSplitK = 32;  // k of one stage of the wide kernel
+// Most floats of split-K partial sums: the allocation-free entry point's
+// scratch, so a plan that splits always fits it.
+constexpr long long kMaxPartialFloats = 8LL << 20;
 // `partial` / `partial_floats`: the caller's buffer for split-K partial
 // sums (nothing is allocated; a plan that needs more is refused); null: the
 // runtime's work buffer, grown as needed.

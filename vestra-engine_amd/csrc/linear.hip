@@ -2,61 +2,71 @@
 // FC1, FC2) with their per-token epilogues (bias, LayerScale, GELU,
 // residual add) fused into the store.
 //
-// A workgroup owns a TM x TN output tile (128 x 128 with 512 threads, or
-// 64 x 128 / 64 x 64 with 256 for grids of few rows); wave w computes rows
-// 32 (w/2) .. +32 and columns TN/2 (w%2) .. +TN/2 as 2 x TN/32 tiles of
-// v_mfma_f32_16x16x4_f32 (F32 in, F32 accumulate): for 128-wide tiles 32
-// MFMAs per 16-wide k-block from six 128-bit LDS reads.  K is staged through
-// LDS in chunks of 64 by raw buffer loads (a lane's fixed offset plus the
-// chunk's uniform offset), A as [m][k] and B as [n][k] rows with a pitch of
-// 68 floats (4 x odd: the 16 rows of a fragment read start on 16 distinct
-// 4-bank groups, and the staging stores of 16 lanes fill one row without
-// conflicts).  The 70 KB of LDS of a 128 x 128 tile leaves room for a
-// second workgroup on the CU, which computes while the first stages a chunk
-// or runs its epilogue.  Grids of few tiles split K over several workgroups
-// per tile (split-K: partial sums in the runtime's work buffer, added in
-// split order by splitk_reduce_kernel).
+// The products run on the f16 matrix cores as three products of two-part
+// splits (split_f16.h), F32 in, F32 accumulate.
 //
-// Fragment order as in the patch embedding: in block b, lane group g holds
-// k = 16b + 4g + j in component j of a 128-bit read and MFMA step j uses
-// component j, so four steps cover the block's 16 k once.
+// A 256-thread workgroup owns a TM x TN output tile (128 x 128; 64 x 128 or
+// 64 x 64 for grids of few rows); wave w computes all TM rows of columns
+// TN/4 w .. + TN/4 as TM/16 x TN/64 tiles of v_mfma_f32_16x16x32_f16.
+//
+//  * A (activations, f32) is read by raw buffer loads one stage ahead, split
+//    by the thread that loaded it and staged through LDS as [row][part][32 k]
+//    f16 rows with a pitch of 144 bytes (16 x odd: the 16 rows of a fragment
+//    read start on 16 distinct 4-bank groups).  Two buffers: one barrier a
+//    stage.
+//  * B (weights) was split when the linear was prepared, each column scaled
+//    by a power of two, into fragment order (split_weights): a wave's operand
+//    of one 16-column tile and part is 1 KiB that its 64 lanes read in order,
+//    straight into registers, one stage ahead.  The waves of a workgroup own
+//    different columns, so no operand of B is read twice and B takes no LDS
+//    space or bandwidth.
+//
+// A 128 x 128 tile runs 48 MFMAs a wave (768 cycles) per 32 k on 8 x 2
+// fragment reads from LDS (4 waves: 512 cycles of its 128 bytes a clock)
+// and 16 + 16 KiB from L2; two workgroups a CU cover each other's barriers.
+// Grids of few tiles split K over several workgroups per tile (split-K:
+// partial sums in the runtime's work buffer, added in split order by
+// splitk_reduce_kernel).
 //
 // Head-major layouts (head_dim 64): the QKV projection can store Q | K | V
 // straight into three [heads, rows, 64] tensors (the split the attention
 // kernels need), and the output projection can read its input from the
 // head-major attention output; tiles start on 64-column head boundaries,
-// and a float4 of A never crosses a head.  Both are pure address changes:
-// the results are the bits of the linear plus the separate permutation.
+// and 32 k of A never cross a head.  Both are pure address changes: the
+// results are the bits of the linear plus the separate permutation.
 //
 // Q/K-norm + RoPE in the QKV epilogue (QKN != 0): after the last chunk the
-// waves holding Q or K heads write their values (acc + b) to LDS and read
-// them back as the Q/K kernel holds a row -- 16 lanes per 64-wide row, one
-// float4 each -- and apply the same row transform (vkq::qk_row_transform)
-// before storing the row head-major.  The values and the code path are
-// those of the separate pass, so the bits are too.
+// waves holding Q or K heads write their values (acc + b) to LDS, 64 rows at
+// a time, and read them back as the Q/K kernel holds a row -- 16 lanes per
+// 64-wide row, one float4 each -- and apply the same row transform
+// (vkq::qk_row_transform) before storing the row head-major.  The values and
+// the code path are those of the separate pass, so the bits are too.
 //
-// Traffic: a 128 x 128 tile moves (128 + 128) x 4 bytes of operands per k for
-// 2 x 128 x 128 FLOP, 0.031 byte per FLOP from L2 (the 48 x 64 tiles of the
-// narrow kernel need 0.073).  Tiles are numbered XCD-major (xcd_tile), so
-// the workgroups of one XCD share weight columns in that XCD's L2.
+// A tile that the split cannot hold (a sum that is not finite, or a row whose
+// values are all tiny, split_f16.h) is computed again by the same workgroup
+// with F32 matrix instructions on the f32 operands.  A split-K workgroup
+// decides for its own run of k.
+//
+// Tiles are numbered XCD-major in groups of at most 1,024 rows (tile_of): the
+// workgroups an XCD holds at one time then share both a slice of A and one
+// of the weights in its L2.
 #include "common.h"
 #include "qk_rows.h"
+#include "split_f16.h"
 
 namespace {
 
 using vk::LinearArgs;
 using namespace vk::linear_epilogue;
+using vks::f32x4;
+using vks::u32x4;
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// Tiles are TM x TN (TM 128 or 64, TN 128 or 64, template parameters); a
-// wave owns a 32-row x TN/2-column strip.
-constexpr int KC = 64;
-constexpr int PITCH = 68;
-static_assert(PITCH % 4 == 0 && (PITCH / 4) % 2 == 1 && PITCH >= KC, "pitch 4 x odd");
-
-// Threads of a TM x 128 tile: one wave per 32 x 64 strip.
-constexpr int threads_for(int tm) { return 4 * tm; }
+constexpr int KC = vk::kSplitK;    // k of one stage (and of one MFMA)
+constexpr int kParts = 2;           // f16 parts of a weight
+constexpr int kThreads = 256;      // four waves
+constexpr int kRowBytes = 144;     // LDS pitch of a row of A: 2 parts x 64 bytes + 16
+constexpr int kXsPitch = 68;       // f32 pitch of the Q/K epilogue's rows
+static_assert(kRowBytes % 16 == 0 && (kRowBytes / 16) % 2 == 1 && kRowBytes >= 4 * KC, "pitch");
 
 enum Layout { kPlain = 0, kQkvHnd = 1, kAHnd = 2 };
 
@@ -133,8 +143,8 @@ __device__ __forceinline__ float4 qk_head_row(const LinearArgs& g, float4 v, int
       v, l, gm, bt, py, px, g.qkn.table, g.qkn.table_max, g.qkn.eps);
 }
 
-// Most split-K slices a sum pass reads (the plan's limit, checked where it
-// is defined).  The sum passes are instantiated for split-count buckets SPB
+// Most split-K slices a sum pass reads (choose_plan and
+// slices_to_provide).  The sum passes are instantiated for split-count buckets SPB
 // of 2, 4 and 8 (split_bucket).
 constexpr int kMaxSplits = 8;
 constexpr int split_bucket(int splits) { return splits <= 2 ? 2 : (splits <= 4 ? 4 : 8); }
@@ -165,346 +175,362 @@ __device__ __forceinline__ void split_sums(const float* __restrict__ partial, si
   }
 }
 
-// KG: k groups.  With KG = 2 (64 x 64 tiles only) the workgroup has twice the
-// waves: group 1 runs the second half of every chunk's 16-blocks on the same
-// strips as group 0, and adds its sums to group 0's through LDS after the
-// last chunk (group 0's + group 1's, in that order).  A grid of few tiles
-// (one image: two workgroups per CU) then keeps four waves per SIMD instead
-// of two.
-//
-// PF: the next chunk's loads are issued before this chunk's MFMAs and land in
-// registers meanwhile.  It costs 2 (64 x 64) or 8 (128 x 128) more float4 per
-// thread, so the 128 x 128 tile takes it only where a launch has at most one
-// workgroup per CU (nothing else on the CU covers the load latency there,
-// and the lower occupancy costs nothing).
-template <int EPI, int LAY, int QKN, int TM, int TN, int KG = 1, bool PF = (KG == 2)>
-__global__ __launch_bounds__(threads_for(TM) * KG,
-                             TM == 128 ? (PF ? 1 : 2) : (TN == 128 ? 3 : (KG == 2 ? 3 : 4)))
-    void linear_wide_kernel(LinearArgs g) {
-  constexpr int WN = TN / 2;  // columns of a wave's strip
-  constexpr int NU = WN / 16; // 16-column MFMA tiles per strip
-  static_assert(TN == 128 || TN == 64, "tile widths 128 and 64");
-  static_assert(KG == 1 || (KG == 2 && TM == 64 && TN == 64), "k groups: 64 x 64 tiles");
-  constexpr int kThreads = threads_for(TM) * KG;
-  constexpr int kGroupWaves = threads_for(TM) / 64;  // waves of one k group
-  constexpr int kVA = TM * KC / 4 / kThreads;  // float4 of A per thread a chunk: 4
-  constexpr int kVB = TN * KC / 4 / kThreads;  // float4 of B: TN / TM x 4
+// The tile and split of workgroup `t`: groups of at most 1,024 rows, in a
+// group split-major, then column tiles, then the group's row tiles (fastest).
+template <int TM>
+__device__ __forceinline__ void tile_of(int t, int gmt, int gnt, int splits, int* mt, int* nt,
+                                        int* split) {
+  constexpr int kGroup = 1024 / TM;
+  const int per_group = kGroup * gnt * splits;
+  const int grp = t / per_group, r = t - grp * per_group;
+  const int left = gmt - grp * kGroup;
+  const int rows = left < kGroup ? left : kGroup;
+  *mt = grp * kGroup + r % rows;
+  const int rest = r / rows;
+  *nt = rest % gnt;
+  *split = rest / gnt;
+}
+
+// KS: stages of 32 k per barrier (2 for the 64-row tiles, whose 12 or 24
+// MFMAs a wave and stage are too few to cover a load's latency).
+template <int EPI, int LAY, int QKN, int TM, int TN, int KS>
+__global__ __launch_bounds__(kThreads, 2) void linear_wide_kernel(LinearArgs g) {
   static_assert(TM == 128 || TM == 64, "tile heights 128 and 64");
-  static_assert(kVA * kThreads * 4 == TM * KC && kVB * kThreads * 4 == TN * KC, "slots");
-  __shared__ __align__(16) float As[TM * PITCH];
-  __shared__ __align__(16) float Bs[TN * PITCH];
+  static_assert(TN == 128 || TN == 64, "tile widths 128 and 64");
+  constexpr int WN = TN / 4;            // columns of a wave
+  constexpr int MT = TM / 16;           // 16-row MFMA tiles of a wave
+  constexpr int NU = WN / 16;           // 16-column MFMA tiles of a wave
+  constexpr int kSlots = TM * 4 * KS;   // 8-k pieces of A a barrier
+  constexpr int kVA = kSlots / kThreads;
+  static_assert(kVA * kThreads == kSlots, "slots divide evenly");
+  constexpr int kStageBytes = TM * kRowBytes;
+  constexpr int kBufBytes = KS * kStageBytes;
+  constexpr int kXsBytes = QKN != 0 ? (TN / 64) * 64 * kXsPitch * 4 : 0;
+  constexpr int kSmem = 2 * kBufBytes > kXsBytes ? 2 * kBufBytes : kXsBytes;
+  __shared__ __align__(16) char smem[kSmem];
 
   const int tid = threadIdx.x;
   __builtin_assume(tid < kThreads);
   const int wave = tid >> 6, lane = tid & 63;
-  const int kh = KG == 1 ? 0 : wave / kGroupWaves;  // k group
-  const bool lead = kh == 0;                          // holds the tile's sums at the end
-  const int wl = wave % kGroupWaves;                  // wave within the k group
-  const int wm = wl >> 1, wn = wl & 1;
   const int gmt = (g.M + TM - 1) / TM;
   const int gnt = (g.N + TN - 1) / TN;
-  const int tile = vkd::xcd_tile(blockIdx.x, gridDim.x);
-  const int m0 = (tile % gmt) * TM;
-  const int rest = tile / gmt;
-  const int n0 = (rest % gnt) * TN;
-  const int split = rest / gnt;
+  int mt, nt, split;
+  tile_of<TM>(vkd::xcd_tile(blockIdx.x, gridDim.x), gmt, gnt, g.splits, &mt, &nt, &split);
+  const int m0 = mt * TM, n0 = nt * TN;
   const int nch = (g.K + KC - 1) / KC;
-  const int c_begin = split * nch / g.splits, c_end = (split + 1) * nch / g.splits;
+  const int c_begin = static_cast<int>(static_cast<long long>(split) * nch / g.splits);
+  const int c_end = static_cast<int>(static_cast<long long>(split + 1) * nch / g.splits);
 
-  f32x4 acc[2][NU];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int u = 0; u < NU; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int kq = 4 * (lane >> 4) + kh * (KC / KG);
-  const float* arow = As + (wm * 32 + (lane & 15)) * PITCH + kq;
-  const float* brow = Bs + (wn * WN + (lane & 15)) * PITCH + kq;
-
-  // Staging slot i of a thread: row r_i = tid/16 + (threads/16) i of the A
-  // (or B) tile, float4 column c = 4 (tid % 16) of the chunk (a wave reads
-  // four 256-byte row segments).  Rows past M or N read a clamped, valid
-  // row: row i of A only reaches output row i and row j of B output column
-  // j, so their values never reach a stored output.
-  const int c_ld = 4 * (tid & 15);
-  uint32_t a_off[kVA], b_off[kVB];  // byte offsets, the same for every chunk
-  auto slot_row = [&](int i) { return (tid >> 4) + (kThreads / 16) * i; };
+  // A: slot i of a thread is piece s = tid + 256 i: stage s / (4 TM), row
+  // (s / 4) % TM, k 8 (s % 4) .. + 8 of that stage.  Rows past M read a
+  // clamped, valid row, which only reaches output rows past M.
+  const int piece = tid & 3;
+  auto slot_row = [&](int i) { return ((tid + kThreads * i) >> 2) % TM; };
+  auto slot_stage = [&](int i) { return (kThreads * i) / (4 * TM); };
+  uint32_t a_off[kVA];
 #pragma unroll
   for (int i = 0; i < kVA; ++i) {
     const int gm = m0 + slot_row(i);
     const uint32_t cm = static_cast<uint32_t>(gm < g.M ? gm : g.M - 1);
-    a_off[i] = 4u * (LAY == kAHnd ? cm * 64u + c_ld : cm * static_cast<uint32_t>(g.K) + c_ld);
+    a_off[i] = 4u * (cm * (LAY == kAHnd ? 64u : static_cast<uint32_t>(g.K)) + 8u * piece);
   }
-#pragma unroll
-  for (int i = 0; i < kVB; ++i) {
-    const int gn = n0 + slot_row(i);
-    const uint32_t cn = static_cast<uint32_t>(gn < g.N ? gn : g.N - 1);
-    b_off[i] = 4u * (cn * static_cast<uint32_t>(g.Kp) + c_ld);
-  }
-
-  auto mma_chunk = [&]() {
-#pragma unroll
-    for (int b = 0; b < KC / 16 / KG; ++b) {
-      f32x4 a[2], w[NU];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-        a[t] = *reinterpret_cast<const f32x4*>(arow + t * 16 * PITCH + 16 * b);
-#pragma unroll
-      for (int u = 0; u < NU; ++u)
-        w[u] = *reinterpret_cast<const f32x4*>(brow + u * 16 * PITCH + 16 * b);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int u = 0; u < NU; ++u)
-            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][j], w[u][j], acc[t][u], 0, 0, 0);
-    }
+  const uint32_t a_bytes = 4u * static_cast<uint32_t>(g.M) * static_cast<uint32_t>(g.K);
+  const __amdgpu_buffer_rsrc_t a_rsrc = vkd::buffer_rsrc(g.x, a_bytes);
+  // byte offset of stage ch for every row
+  auto a_chunk = [&](int ch) {
+    return LAY == kAHnd ? 4u * (static_cast<uint32_t>(ch >> 1) * static_cast<uint32_t>(g.M) * 64u +
+                                static_cast<uint32_t>(ch & 1) * 32u)
+                        : 4u * static_cast<uint32_t>(ch) * KC;
   };
-
-  // Whole chunks (k0 + 64 <= K): buffer loads of the lane's fixed offset
-  // plus the chunk's uniform offset, with no per-chunk address arithmetic or
-  // selects.
-  const int full = g.K / KC;
-  const int c_full = c_end < full ? c_end : full;
-  const __amdgpu_buffer_rsrc_t a_rsrc =
-      vkd::buffer_rsrc(g.x, 4u * static_cast<uint32_t>(g.M) * static_cast<uint32_t>(g.K));
-  const __amdgpu_buffer_rsrc_t b_rsrc =
-      vkd::buffer_rsrc(g.wnk, 4u * static_cast<uint32_t>(g.N) * static_cast<uint32_t>(g.Kp));
-  auto load_chunk = [&](int ch, float4 (&ra)[kVA], float4 (&rb)[kVB]) {
-    const uint32_t k0 = static_cast<uint32_t>(ch) * KC;
-    const uint32_t a_chunk =
-        4u * (LAY == kAHnd ? static_cast<uint32_t>(ch) * static_cast<uint32_t>(g.M) * 64u : k0);
-#pragma unroll
-    for (int i = 0; i < kVA; ++i) ra[i] = vkd::buffer_load4(a_rsrc, a_off[i], a_chunk);
-#pragma unroll
-    for (int i = 0; i < kVB; ++i) rb[i] = vkd::buffer_load4(b_rsrc, b_off[i], 4u * k0);
-  };
-  auto store_chunk = [&](const float4 (&ra)[kVA], const float4 (&rb)[kVB]) {
-#pragma unroll
-    for (int i = 0; i < kVA; ++i)
-      *reinterpret_cast<float4*>(As + slot_row(i) * PITCH + c_ld) = ra[i];
-#pragma unroll
-    for (int i = 0; i < kVB; ++i)
-      *reinterpret_cast<float4*>(Bs + slot_row(i) * PITCH + c_ld) = rb[i];
-  };
-  if constexpr (PF) {
-    float4 ra[kVA], rb[kVB];
-    if (c_begin < c_full) load_chunk(c_begin, ra, rb);
-    for (int ch = c_begin; ch < c_full; ++ch) {
-      __syncthreads();  // every wave is done reading the previous chunk
-      store_chunk(ra, rb);
-      __syncthreads();
-      if (ch + 1 < c_full) load_chunk(ch + 1, ra, rb);
-      mma_chunk();
-    }
-  } else {
-    for (int ch = c_begin; ch < c_full; ++ch) {
-      float4 ra[kVA], rb[kVB];
-      load_chunk(ch, ra, rb);
-      __syncthreads();  // every wave is done reading the previous chunk
-      store_chunk(ra, rb);
-      __syncthreads();
-      mma_chunk();
-    }
-  }
-
-  // The last, partial chunk (K % 64 != 0): k past K reads a clamped address
-  // and stores zeros (A past K, B past its zero padding Kp).
-  if (c_end > full && c_begin <= full) {
-    const int k0 = full * KC;
-    const int gk = k0 + c_ld;
-    const bool ka = gk < g.K, kb = gk < g.Kp;
-    const int ck = ka ? gk : g.K - 4;
-    const int ckb = kb ? gk : g.Kp - 4;
-    float4 ra[kVA], rb[kVB];
+  float4 ra[kVA][2];
+  // k past K, and stages past the split's end, read past the buffer, which
+  // gives zeros.
+  auto load_a = [&](int ch0) {
 #pragma unroll
     for (int i = 0; i < kVA; ++i) {
-      const int gm = m0 + slot_row(i);
-      const int cm = gm < g.M ? gm : g.M - 1;
-      const size_t ia = LAY == kAHnd
-                            ? (static_cast<size_t>(ck >> 6) * g.M + cm) * 64 + (ck & 63)
-                            : static_cast<size_t>(cm) * g.K + ck;
-      ra[i] = *reinterpret_cast<const float4*>(g.x + ia);
+      const int at = ch0 + slot_stage(i);
+      const int ch = at < c_end ? at : c_end - 1;
+      const int left = at < c_end ? g.K - ch * KC : 0;  // uniform
+      const uint32_t base = a_chunk(ch);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        ra[i][h] = vkd::buffer_load4(
+            a_rsrc, 8 * piece + 4 * h < left ? a_off[i] + 16u * h : 0xfffffff0u, base);
     }
+  };
+  float amax[kVA];  // largest |x| of the slot's pieces so far
 #pragma unroll
-    for (int i = 0; i < kVB; ++i) {
-      const int gn = n0 + slot_row(i);
-      const int cn = gn < g.N ? gn : g.N - 1;
-      rb[i] = *reinterpret_cast<const float4*>(g.wnk + static_cast<size_t>(cn) * g.Kp + ckb);
+  for (int i = 0; i < kVA; ++i) amax[i] = 0.0f;
+  auto store_a = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < kVA; ++i) {
+      amax[i] = vks::max_abs8(amax[i], ra[i][0], ra[i][1]);
+      u32x4 p0, p1;
+      vks::split8(ra[i][0], ra[i][1], &p0, &p1);
+      char* d = smem + buf * kBufBytes + slot_stage(i) * kStageBytes + slot_row(i) * kRowBytes +
+                16 * piece;
+      *reinterpret_cast<u32x4*>(d) = p0;
+      *reinterpret_cast<u32x4*>(d + 64) = p1;
     }
-    __syncthreads();
-    // component selects: a select of whole float4 values becomes a select
-    // of their addresses, which puts the staging arrays in scratch memory
+  };
+
+  // B: 16-column tile j of the weights, stage ch, part p: 64 x 16 bytes at
+  // ((j nch + ch) 2 + p) KiB.  Tiles past N read the last one; their columns
+  // are not stored.
+  const int ntiles = (g.N + 15) / 16;
+  const u32x4* bptr[NU];
 #pragma unroll
-    for (int i = 0; i < kVA; ++i)
-      *reinterpret_cast<float4*>(As + slot_row(i) * PITCH + c_ld) =
-          make_float4(ka ? ra[i].x : 0.f, ka ? ra[i].y : 0.f, ka ? ra[i].z : 0.f,
-                      ka ? ra[i].w : 0.f);
+  for (int u = 0; u < NU; ++u) {
+    const int j = (n0 + wave * WN) / 16 + u;
+    const int cj = j < ntiles ? j : ntiles - 1;
+    bptr[u] = reinterpret_cast<const u32x4*>(g.wsplit) +
+              static_cast<size_t>(cj) * nch * (kParts * 64) + lane;
+  }
+  auto load_b = [&](int ch0, u32x4 (&b)[KS][NU][kParts]) {
 #pragma unroll
-    for (int i = 0; i < kVB; ++i)
-      *reinterpret_cast<float4*>(Bs + slot_row(i) * PITCH + c_ld) =
-          make_float4(kb ? rb[i].x : 0.f, kb ? rb[i].y : 0.f, kb ? rb[i].z : 0.f,
-                      kb ? rb[i].w : 0.f);
+    for (int s = 0; s < KS; ++s) {
+      // a stage past the split's end multiplies zeros of A
+      const int ch = ch0 + s < c_end ? ch0 + s : c_end - 1;
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int p = 0; p < kParts; ++p)
+          b[s][u][p] = bptr[u][static_cast<size_t>(ch) * (kParts * 64) + p * 64];
+    }
+  };
+  const char* afrag = smem + (lane & 15) * kRowBytes + 16 * (lane >> 4);
+  f32x4 acc[MT][NU], corr[MT][NU];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int u = 0; u < NU; ++u) acc[t][u] = corr[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Fragments of the next 16 rows are read while these rows' MFMAs run.
+  auto mma = [&](int buf, const u32x4 (&b)[KS][NU][kParts]) {
+    u32x4 a[2][2];
+    auto read_a = [&](int st, u32x4 (&f)[2]) {
+      const char* ar = afrag + buf * kBufBytes + (st / MT) * kStageBytes +
+                       (st % MT) * 16 * kRowBytes;
+      f[0] = *reinterpret_cast<const u32x4*>(ar);
+      f[1] = *reinterpret_cast<const u32x4*>(ar + 64);
+    };
+    read_a(0, a[0]);
+#pragma unroll
+    for (int st = 0; st < KS * MT; ++st) {
+      const int s = st / MT, t = st % MT;
+      if (st + 1 < KS * MT) read_a(st + 1, a[(st + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      const u32x4(&f)[2] = a[st & 1];
+#pragma unroll
+      for (int u = 0; u < NU; ++u) acc[t][u] = vks::mfma(f[0], b[s][u][0], acc[t][u]);
+#pragma unroll
+      for (int u = 0; u < NU; ++u) corr[t][u] = vks::mfma(f[0], b[s][u][1], corr[t][u]);
+#pragma unroll
+      for (int u = 0; u < NU; ++u) corr[t][u] = vks::mfma(f[1], b[s][u][0], corr[t][u]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // One stage: split and store what was loaded a stage earlier, issue the
+  // next stage's loads, run this one's MFMAs.  A buffer is written again two
+  // stages after it was read, with a barrier in between.
+  u32x4 b0[KS][NU][kParts], b1[KS][NU][kParts];
+  load_a(c_begin);
+  load_b(c_begin, b0);
+  int ch = c_begin;
+  for (; ch + KS < c_end; ch += 2 * KS) {
+    store_a(0);
     __syncthreads();
-    mma_chunk();
+    load_a(ch + KS);
+    load_b(ch + KS, b1);
+    mma(0, b0);
+    store_a(1);
+    __syncthreads();
+    load_a(ch + 2 * KS);
+    load_b(ch + 2 * KS, b0);
+    mma(1, b1);
+  }
+  if (ch < c_end) {
+    store_a(0);
+    __syncthreads();
+    mma(0, b0);
   }
 
-  // k groups: the two groups' sums meet through LDS (As, free after the
-  // last chunk), one f32x4 per lane and MFMA tile, lane-contiguous.  For the
-  // plain epilogue each group finishes one of the strip's two 16-row halves
-  // (half kh: it hands the other half's sums over and takes this half's),
-  // so all eight waves run the epilogue; the Q/K epilogue and split-K take
-  // the whole sums in group 0.  Either way a sum is group 0's + group 1's.
-  const bool half_epi = KG == 2 && QKN == 0 && g.splits == 1;
-  if constexpr (KG == 2) {
-    static_assert(kGroupWaves * 2 * NU * 256 <= TM * PITCH, "k-group sums fit in As");
-    float* red = As + wl * (2 * NU * 256) + 4 * lane;
-    __syncthreads();  // every wave is done reading the last chunk's operands
-    if (half_epi) {
-      // constant indices in both branches (kh is uniform over the wave): a
-      // register array indexed by a run-time value would live in scratch
-      if (lead) {
+  // lane holds D[4 (lane / 16) + r][lane % 16] of each 16 x 16 tile
+  const int g4 = lane >> 4, c16 = lane & 15;
+  auto row_of = [&](int t, int r) { return m0 + t * 16 + 4 * g4 + r; };
+  auto col_of = [&](int u) { return n0 + wave * WN + u * 16 + c16; };
+
+  // The sums, and whether the split held everything that went into them.
+  bool odd = false;
 #pragma unroll
-        for (int u = 0; u < NU; ++u)
-          *reinterpret_cast<f32x4*>(red + (NU + u) * 256) = acc[1][u];
-      } else {
+  for (int u = 0; u < NU; ++u) {
+    const int e = -g.wexp[col_of(u) < g.N ? col_of(u) : g.N - 1];
 #pragma unroll
-        for (int u = 0; u < NU; ++u) *reinterpret_cast<f32x4*>(red + u * 256) = acc[0][u];
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = __builtin_fmaf(corr[t][u][r], vks::kDown, acc[t][u][r]);
+        odd |= !vks::is_finite(v);
+        acc[t][u][r] = __builtin_amdgcn_ldexpf(v, e);
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < kVA / KS; ++i) {  // the four pieces of a row are adjacent lanes
+    float m = amax[i];
+#pragma unroll
+    for (int s = 1; s < KS; ++s) m = fmaxf(m, amax[i + s * (kVA / KS)]);
+    m = fmaxf(m, __shfl_xor(m, 1, 64));
+    m = fmaxf(m, __shfl_xor(m, 2, 64));
+    odd |= m < vks::kRowMin && m != 0.0f;
+  }
+  int* flags = reinterpret_cast<int*>(smem);  // one per wave
+  __syncthreads();  // every wave is done with the last stage
+  const bool wave_odd = __builtin_amdgcn_ballot_w64(odd) != 0;
+  if (lane == 0) flags[wave] = wave_odd;
+  __syncthreads();
+  if (__builtin_expect(flags[0] | flags[1] | flags[2] | flags[3], 0)) {
+    // The tile again, with F32 matrix instructions (fragment order: lane
+    // group g4 holds k = 16 b + 4 g4 + j of block b in component j).
+    constexpr int kPitchF = kRowBytes / 4;
+    float* As = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < NU; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int ch = c_begin; ch < c_end; ++ch) {
+      __syncthreads();
+#pragma unroll 1
+      for (int s = tid; s < TM * 8; s += kThreads) {
+        const int row = s >> 3, k = ch * KC + 4 * (s & 7);
+        const int gm = m0 + row < g.M ? m0 + row : g.M - 1;
+        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+        const size_t at = LAY == kAHnd ? (static_cast<size_t>(k >> 6) * g.M + gm) * 64 + (k & 63)
+                                       : static_cast<size_t>(gm) * g.K + k;
+        *reinterpret_cast<float4*>(As + row * kPitchF + 4 * (s & 7)) =
+            k < g.K ? *reinterpret_cast<const float4*>(g.x + at) : z;
       }
       __syncthreads();
-      if (lead) {
+#pragma unroll 1
+      for (int b = 0; b < 2; ++b) {
+        const int k = ch * KC + 16 * b + 4 * g4;
+        f32x4 w[NU];
 #pragma unroll
-        for (int u = 0; u < NU; ++u)
-          acc[0][u] = acc[0][u] + *reinterpret_cast<const f32x4*>(red + u * 256);
-      } else {
+        for (int u = 0; u < NU; ++u) {
+          const int col = col_of(u) < g.N ? col_of(u) : g.N - 1;
+          w[u] = k < g.Kp ? *reinterpret_cast<const f32x4*>(g.wnk + static_cast<size_t>(col) * g.Kp + k)
+                          : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
-        for (int u = 0; u < NU; ++u)
-          acc[1][u] = *reinterpret_cast<const f32x4*>(red + (NU + u) * 256) + acc[1][u];
-      }
-    } else {
-      if (!lead) {
+        for (int t = 0; t < MT; ++t) {
+          const f32x4 a =
+              *reinterpret_cast<const f32x4*>(As + (t * 16 + c16) * kPitchF + 16 * b + 4 * g4);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+          for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int u = 0; u < NU; ++u)
-            *reinterpret_cast<f32x4*>(red + (t * NU + u) * 256) = acc[t][u];
-      }
-      __syncthreads();
-      if (lead) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int u = 0; u < NU; ++u)
-            acc[t][u] = acc[t][u] + *reinterpret_cast<const f32x4*>(red + (t * NU + u) * 256);
+            for (int u = 0; u < NU; ++u)
+              acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], w[u][j], acc[t][u], 0, 0, 0);
+        }
       }
     }
   }
 
   // split-K: raw sums to this split's slice of the partial buffer
   if (g.splits > 1) {
-    if (lead) {
-      float* part = g.partial + static_cast<size_t>(split) * g.M * g.N;
+    float* part = g.partial + static_cast<size_t>(split) * g.M * g.N;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int u = 0; u < NU; ++u)
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int row = m0 + wm * 32 + t * 16 + 4 * (lane >> 4) + r;
-            const int col = n0 + wn * WN + u * 16 + (lane & 15);
-            if (row < g.M && col < g.N) part[static_cast<size_t>(row) * g.N + col] = acc[t][u][r];
-          }
-    }
+        for (int u = 0; u < NU; ++u) {
+          const int row = row_of(t, r), col = col_of(u);
+          if (row < g.M && col < g.N) part[static_cast<size_t>(row) * g.N + col] = acc[t][u][r];
+        }
     return;
   }
 
-  // epilogue: lane holds D[4*(lane/16) + r][lane%16] of each 16x16 tile.
-  // Parameters and (for the residual) the old values are all loaded, on
-  // clamped indices, before the first store.
-  float bias[NU], ls[NU];
+  // epilogue.  Parameters and (for the residual) the old values are all
+  // loaded, on clamped indices, before the first store.
   if constexpr (QKN != 0) {
     static_assert(LAY == kQkvHnd && EPI == kLinStore, "Q/K epilogue of the QKV projection");
-    // One head of Q, K or V: a 128-wide tile gives each wave a head of its
-    // own (its 32 x 64 strip); a 64-wide tile is one head, whose 32-row
-    // halves waves wn 0 and 1 hold 32 columns each of and then transform 16
-    // rows each.
-    // With k groups, the eight waves transform 8 rows each.
-    const int col0 = TN == 128 ? n0 + wn * 64 : n0;
-    const int cw0 = TN == 128 ? 0 : wn * 32;  // the wave's first column in the head
-    constexpr int kRowsPerGroup = TN == 128 ? 8 : 4 / KG;
-    const int rr0 = TN == 128 ? 0 : (wn * KG + kh) * (16 / KG);
+    // A head of Q, K or V is two waves of a 128-wide tile or all four of a
+    // 64-wide one; its 64-row halves meet in LDS one after the other.
+    constexpr int kHeadWaves = 256 / TN;              // 2 or 4
+    constexpr int kRowsPerGroup = 16 / kHeadWaves;    // rows of a 16-lane group a half
+    const int head = wave / kHeadWaves, hw = wave % kHeadWaves;
+    const int col0 = n0 + head * 64;
     const int embed = g.N / 3;
     const int which = col0 < g.N ? col0 / embed : 2;
-    const int g4 = lane >> 4, c16 = lane & 15;
-    // 32-row staging regions: TN 128, one per wave (the A tile holds TM / 32
-    // of them, the B tile the rest); TN 64, one per row half wm, in the A tile
-    float* xs = TN == 64 ? As + wm * 32 * PITCH
-                         : (wave < TM / 32 ? As + wave * 32 * PITCH
-                                           : Bs + (wave - TM / 32) * 32 * PITCH);
-    __syncthreads();  // every wave is done with the last chunk's operands
-    if (which < 2 && lead) {
+    float* xs = reinterpret_cast<float*>(smem) + head * 64 * kXsPitch;
+    float* dst = nullptr;
+    if (which < 2)
+      dst = (which == 0 ? g.q_out : g.k_out) +
+            static_cast<size_t>((col0 - which * embed) >> 6) * g.M * 64;
 #pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const float b = g.bias[col0 + cw0 + u * 16 + c16];
+    for (int half = 0; half < TM / 64; ++half) {
+      __syncthreads();  // every wave is done with what LDS held
+      if (which < 2) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int u = 0; u < NU; ++u) {
+          const float b = g.bias[col_of(u)];
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            xs[(t * 16 + 4 * g4 + r) * PITCH + cw0 + u * 16 + c16] = acc[t][u][r] + b;
+          for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              xs[(t * 16 + 4 * g4 + r) * kXsPitch + hw * WN + u * 16 + c16] =
+                  acc[half * 4 + t][u][r] + b;
+        }
       }
-    }
-    __syncthreads();
-    if (which < 2) {
-      float* dst = (which == 0 ? g.q_out : g.k_out) +
-                   static_cast<size_t>((col0 - which * embed) >> 6) * g.M * 64;
+      __syncthreads();
+      if (which < 2) {
 #pragma unroll 2
-      for (int i = 0; i < kRowsPerGroup; ++i) {
-        const int rr = rr0 + g4 * kRowsPerGroup + i;
-        const int row = m0 + wm * 32 + rr;
-        const float4 v = *reinterpret_cast<const float4*>(xs + rr * PITCH + 4 * c16);
-        const float4 o = qk_head_row<QKN>(g, v, c16, which == 1, row);
-        if (row < g.M) *reinterpret_cast<float4*>(dst + static_cast<size_t>(row) * 64 + 4 * c16) = o;
+        for (int i = 0; i < kRowsPerGroup; ++i) {
+          const int rr = (hw * 4 + g4) * kRowsPerGroup + i;
+          const int row = m0 + half * 64 + rr;
+          const float4 v = *reinterpret_cast<const float4*>(xs + rr * kXsPitch + 4 * c16);
+          const float4 o = qk_head_row<QKN>(g, v, c16, which == 1, row);
+          if (row < g.M)
+            *reinterpret_cast<float4*>(dst + static_cast<size_t>(row) * 64 + 4 * c16) = o;
+        }
       }
-      return;
     }
+    if (which < 2) return;
   }
-  if (!lead && !half_epi) return;
   // Per 16-column strip u: bias, LayerScale and the address of the column
   // at row 0 (row r adds r x the row stride), computed once; a tile inside
   // the matrix stores without bounds checks.
   const bool interior = m0 + TM <= g.M && n0 + TN <= g.N;
   const size_t rs = LAY == kQkvHnd ? 64 : static_cast<size_t>(g.N);
+  float bias[NU], ls[NU];
   float* cptr[NU];
   bool cok[NU];
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int col = n0 + wn * WN + u * 16 + (lane & 15);
+    const int col = col_of(u);
     cok[u] = col < g.N;
     const int cc = cok[u] ? col : g.N - 1;
     bias[u] = g.bias[cc];
     ls[u] = g.ls ? g.ls[cc] : 1.0f;
     cptr[u] = out_addr<LAY>(g, 0, cc);
   }
-  float old[2][NU][4];
+  float old[MT][NU][4];
   if constexpr (EPI == kLinResidual) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        if (half_epi && t != kh) continue;
-        const int row = m0 + wm * 32 + t * 16 + 4 * (lane >> 4) + r;
+        const int row = row_of(t, r);
         const size_t cr = static_cast<size_t>(row < g.M ? row : g.M - 1);
 #pragma unroll
         for (int u = 0; u < NU; ++u) old[t][u][r] = cptr[u][cr * rs];
       }
   }
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      if (half_epi && t != kh) continue;
-      const int row = m0 + wm * 32 + t * 16 + 4 * (lane >> 4) + r;
+      const int row = row_of(t, r);
       const bool rok = row < g.M;
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
@@ -625,33 +651,6 @@ namespace vk {
 
 namespace {
 
-// Tile shape and split count, from a cost model fitted to plan sweeps of
-// the ViT-B and ViT-L projections at 866 and 3,458 rows.  Workgroups are
-// dealt round-robin to the CUs, so the busiest CU runs ceil(tiles * s / CUs)
-// workgroups of up to ceil(chunks / s) K chunks each: about 5.5 us per
-// chunk of a 128 x 128 tile, 0.6 of that for 64 x 128 and 0.28 for 64 x 64
-// (a quarter of the MFMAs, more operand staging per MFMA, and more
-// workgroups per CU to hide it: 1.0-1.5 us measured).  A split adds its
-// partial sums (s x M x N floats written, then read by the sum pass, at
-// about 5.5 TB/s) and the sum pass's launch (about 2 us).  The cheapest plan
-// wins; on ties the larger tile, then the smaller count.  At least two
-// chunks per split, at most VK_SPLITK_MAX slices and VK_SPLITK_MAX_FLOATS
-// floats of partial sums.  One 866-token ViT-B image: QKV and FC1 64 x 64
-// unsplit, projection 64 x 64 x 3, FC2 128 x 128 x 6; ViT-L at 3,458 rows:
-// FC1 64 x 64, the others 128 x 128 (FC2 x 8); 10,392 rows: 128 x 128
-// unsplit.
-#ifndef VK_SPLITK_MAX
-#define VK_SPLITK_MAX 8  // most partial slices
-#endif
-static_assert(VK_SPLITK_MAX >= 1 && VK_SPLITK_MAX <= kMaxSplits,
-              "the sum passes read at most kMaxSplits slices");
-#ifndef VK_SPLITK_MAX_FLOATS
-#define VK_SPLITK_MAX_FLOATS (1LL << 26)  // 256 MB of partial sums
-#endif
-#ifndef VK_LINEAR_TILES
-#define VK_LINEAR_TILES 7  // allowed tiles: bit 0 128x128, bit 1 64x128, bit 2 64x64
-#endif
-
 struct Plan {
   int tm, tn;
   int splits;
@@ -662,27 +661,85 @@ long long tile_count(int tm, int tn, int M, int N) {
   return static_cast<long long>((M + tm - 1) / tm) * static_cast<long long>((N + tn - 1) / tn);
 }
 
-Plan choose_plan(const vk_runtime* rt, int M, int N, int K) {
+// Partial slices a caller must be ready to provide for: 1 where the shape
+// never splits (it can be captured before any eager call of its kind), else
+// the count that the allocation-free entry point's scratch is held against.
+// This is the interface's rule, fixed apart from what a plan takes (a plan
+// never takes more floats than this count, or kMaxPartialFloats): the
+// cheapest of 128 x 128, 64 x 128 and 64 x 64 tiles in runs of 64-wide K
+// chunks, at 5.5 us per chunk of the busiest CU's 128 x 128 tiles (0.6 and
+// 0.28 of that for the others) plus the partial sums' traffic at 5.5 TB/s
+// and 2 us for the sum pass; on ties the larger tile, then the smaller count.
+int slices_to_provide(long long cus, int M, int N, int K) {
   constexpr double kChunkUs = 5.5, kBytesPerUs = 5.5e6, kSumLaunchUs = 2.0;
-  // tile shape, cost of one of its K chunks relative to a 128 x 128 chunk
   struct Shape {
-    int tm, tn, bit;
+    int tm, tn;
     double cost;
   };
-  constexpr Shape kShapes[] = {{128, 128, 1, 1.0}, {64, 128, 2, 0.6}, {64, 64, 4, 0.28}};
-  const long long cus = rt->cu_count > 0 ? rt->cu_count : 256;
-  const int nch = (K + KC - 1) / KC;
+  constexpr Shape kShapes[] = {{128, 128, 1.0}, {64, 128, 0.6}, {64, 64, 0.28}};
+  const int nch = (K + 63) / 64;
   const long long mn = static_cast<long long>(M) * N;
-  Plan best{0, 0, 1, 0};
+  int best = 0;
   double best_us = 0.0;
   for (const Shape& sh : kShapes) {
-    if (!(VK_LINEAR_TILES & sh.bit)) continue;
     const long long tiles = tile_count(sh.tm, sh.tn, M, N);
-    for (int sp = 1; sp == 1 || (sp <= VK_SPLITK_MAX && 2 * sp <= nch &&
-                                 sp * mn <= VK_SPLITK_MAX_FLOATS);
+    for (int sp = 1; sp == 1 || (sp <= kMaxSplits && 2 * sp <= nch && sp * mn <= (1LL << 26));
          ++sp) {
       const long long load = (tiles * sp + cus - 1) / cus * ((nch + sp - 1) / sp);
       double us = kChunkUs * sh.cost * static_cast<double>(load);
+      if (sp > 1) us += 8.0 * static_cast<double>(sp * mn) / kBytesPerUs + kSumLaunchUs;
+      if (best == 0 || us < best_us) {
+        best = sp;
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
+// Tile shape and split count, from a cost model fitted to plan sweeps of
+// the ViT-B and ViT-L projections at 100 to 10,392 rows.  Workgroups are
+// dealt round-robin to the CUs, so the busiest CU runs ceil(tiles * s / CUs)
+// workgroups of up to ceil(stages / s) 32-wide K stages each: 0.85 us per
+// stage of a 128 x 128 tile, 0.43 of a 64 x 128 and 0.26 of a 64 x 64 one (a
+// quarter of the MFMAs on half the operands); a CU with one workgroup has
+// nothing to cover its waits and counts 1.3.  A split adds its partial sums
+// (s x M x N floats written, then read by the sum pass, at about 5.5 TB/s)
+// and the sum pass's launch (about 2 us).  The cheapest plan wins; on ties
+// the larger tile, then the smaller count.  At least four stages per split;
+// where the shape may split, at most kMaxStages of them (a run's rounding
+// grows with its length: K = 4096, 4.1e-7 of the 64-bit result unsplit, 3.0e-7
+// in two).  Measured (model's choice; neighbours): 866 x 768 -> 2304, 64 x 64
+// 18.3 us (64 x 128 19.3, 128 x 128 28); 866 x 3072 -> 768, 64 x 64 x 3 24.7
+// (unsplit 35, 64 x 128 x 6 24.4); 1500 x 768 -> 2304, 64 x 128 26.0 (64 x 64
+// 29.6, 128 x 128 31.5); 10,392 x 3072 -> 768, 128 x 128 155 (64 x 128 161, 64
+// x 64 198).
+constexpr int kMaxStages = 96;
+
+Plan choose_plan(long long cus, int M, int N, int K, int provided) {
+  constexpr double kBytesPerUs = 5.5e6, kSumLaunchUs = 2.0, kAlone = 1.3;
+  // tile shape, us of one of its K stages
+  struct Shape {
+    int tm, tn;
+    double us;
+  };
+  constexpr Shape kShapes[] = {{128, 128, 0.85}, {64, 128, 0.43}, {64, 64, 0.26}};
+  const int nch = (K + KC - 1) / KC;
+  const long long mn = static_cast<long long>(M) * N;
+  // the shortest run is kMaxStages or, if the slices do not allow that, 1 / max
+  const auto may = [&](int sp) {
+    return sp == 1 || (provided > 1 && sp <= kMaxSplits && 4 * sp <= nch &&
+                       (sp <= provided || sp * mn <= kMaxPartialFloats));
+  };
+  Plan best{0, 0, 1, 0};
+  double best_us = 0.0;
+  for (const Shape& sh : kShapes) {
+    const long long tiles = tile_count(sh.tm, sh.tn, M, N);
+    for (int sp = 1; may(sp); ++sp) {
+      const int stages = (nch + sp - 1) / sp;
+      if (stages > kMaxStages && may(sp + 1)) continue;
+      const double load = static_cast<double>((tiles * sp + cus - 1) / cus);
+      double us = sh.us * stages * (load > 1.0 ? load : kAlone);
       if (sp > 1) us += 8.0 * static_cast<double>(sp * mn) / kBytesPerUs + kSumLaunchUs;
       if (best.tm == 0 || us < best_us) {
         best = Plan{sh.tm, sh.tn, sp, tiles};
@@ -696,19 +753,15 @@ Plan choose_plan(const vk_runtime* rt, int M, int N, int K) {
 template <int EPI, int LAY, int QKN = 0>
 void launch_pair(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 grid,
                  bool sum_pass = true) {
-  const long long cus = rt->cu_count > 0 ? rt->cu_count : 256;
-  if (plan.tm == 128 && static_cast<long long>(grid.x) <= cus)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 128, 1, true>), grid,
-                       dim3(threads_for(128)), 0, rt->stream, g);
-  else if (plan.tm == 128)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 128>), grid,
-                       dim3(threads_for(128)), 0, rt->stream, g);
+  if (plan.tm == 128)
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 128, 1>), grid, dim3(kThreads), 0,
+                       rt->stream, g);
   else if (plan.tn == 128)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 128>), grid, dim3(threads_for(64)),
-                       0, rt->stream, g);
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 128, 2>), grid, dim3(kThreads), 0,
+                       rt->stream, g);
   else
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 64, 2>), grid,
-                       dim3(2 * threads_for(64)), 0, rt->stream, g);
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 64, 2>), grid, dim3(kThreads), 0,
+                       rt->stream, g);
   if (g.splits > 1 && sum_pass) {
     const long long n4 = static_cast<long long>(g.M) * g.N / 4;
     const dim3 sgrid(static_cast<unsigned>((n4 + 255) / 256));
@@ -731,31 +784,105 @@ void launch_pair(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 gri
 
 }  // namespace
 
+// Exponent of each weight column for the split: wexp[n] = e brings the
+// column's largest |w| to 2^e |w| in [2^10, 2^11), so that every value down to
+// 2^-24 of it has both parts (0 for a column of zeros).
+__global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __restrict__ wnk,
+                                                              int* __restrict__ wexp, int N,
+                                                              int Kp) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= N) return;
+  uint32_t m = 0;
+  for (int k = lane; k < Kp; k += 64) {
+    const uint32_t b = __float_as_uint(wnk[static_cast<size_t>(row) * Kp + k]) & 0x7fffffffu;
+    if (b < 0x7f800000u) m = b > m ? b : m;
+  }
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    const uint32_t o = __shfl_xor(m, s, 64);
+    m = o > m ? o : m;
+  }
+  int e = 0;
+  if (m) (void)frexpf(__uint_as_float(m), &e);  // m in [2^(e-1), 2^e)
+  if (lane == 0) wexp[row] = m ? 11 - e : 0;
+}
+
+// The f16 parts of the scaled rows 2^wexp[n] wnk[n] of [N, Kp] in the order
+// the wide kernel's lanes read them: 16-row tile j, 32-k stage ch, part p,
+// lane l (row 16 j + l % 16, k 32 ch + 8 (l / 16) .. + 8), 16 bytes each.
+// Rows past N and k past Kp are zeros.
+__global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ wnk,
+                                                            const int* __restrict__ wexp,
+                                                            u32x4* __restrict__ dst, int N, int Kp,
+                                                            int nch, long long pieces) {
+  const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= pieces) return;
+  const int lane = static_cast<int>(i & 63);
+  const long long jc = i >> 6;
+  const int ch = static_cast<int>(jc % nch);
+  const long long row = (jc / nch) * 16 + (lane & 15);
+  const int k0 = ch * KC + 8 * (lane >> 4);
+  const int e = row < N ? wexp[row] : 0;
+  auto at = [&](int h) {
+    return row < N && k0 + h < Kp ? ldexpf(wnk[static_cast<size_t>(row) * Kp + k0 + h], e) : 0.0f;
+  };
+  u32x4 p0, p1;
+  vks::split8(make_float4(at(0), at(1), at(2), at(3)), make_float4(at(4), at(5), at(6), at(7)), &p0,
+              &p1);
+  dst[jc * 128 + lane] = p0;
+  dst[jc * 128 + 64 + lane] = p1;
+}
+
+int split_weights(vk_linear* lin) {
+  if (lin->in_features % 4 != 0) return VK_OK;  // never on the wide kernel
+  const long long ntiles = (static_cast<long long>(lin->out_features) + 15) / 16;
+  const long long nch = (static_cast<long long>(lin->in_features) + KC - 1) / KC;
+  const long long pieces = ntiles * nch * 64;
+  const long long blocks = (pieces + 255) / 256;
+  VK_UNSUPPORTED_IF(blocks > 0x7fffffffLL, "linear too large");
+  const int n = static_cast<int>(lin->out_features), kp = static_cast<int>(lin->k_pitch);
+  // one allocation: the parts, then the exponents
+  const size_t bytes = static_cast<size_t>(pieces) * 32;
+  VK_HIP(hipMalloc(&lin->weight_split, bytes + static_cast<size_t>(n) * sizeof(int)));
+  lin->weight_exp = reinterpret_cast<int*>(static_cast<char*>(lin->weight_split) + bytes);
+  hipLaunchKernelGGL(weight_exponent_kernel, dim3((n + 3) / 4), dim3(256), 0, nullptr,
+                     lin->weight_nk, lin->weight_exp, n, kp);
+  VK_TRY(check_launch("weight_exponent_kernel"));
+  hipLaunchKernelGGL(split_weights_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
+                     nullptr, lin->weight_nk, lin->weight_exp,
+                     static_cast<u32x4*>(lin->weight_split), n, kp, static_cast<int>(nch), pieces);
+  VK_TRY(check_launch("split_weights_kernel"));
+  VK_HIP(hipStreamSynchronize(nullptr));
+  return VK_OK;
+}
+
 int launch_linear_wide(vk_runtime* rt, const LinearArgs& g0, int epi, float* partial,
                        size_t partial_floats) {
   LinearArgs g = g0;
-  // An output element's bits depend on the plan (its split count, and the
-  // two k groups of a 64 x 64 tile, added at the end) and the plan on
-  // (M, N, K) alone, so every layout and epilogue of one shape gives the
-  // same bits.
-  const Plan plan = choose_plan(rt, g.M, g.N, g.K);
+  // An output element's bits depend on the plan (its split count) and the
+  // plan on (M, N, K) alone, so every layout and epilogue of one shape gives
+  // the same bits.
+  const long long cus = rt->cu_count > 0 ? rt->cu_count : 256;
+  const int provided = slices_to_provide(cus, g.M, g.N, g.K);
+  const Plan plan = choose_plan(cus, g.M, g.N, g.K, provided);
   g.splits = plan.splits;
   g.partial = nullptr;
   VK_UNSUPPORTED_IF(plan.tiles * g.splits > 0x7fffffffLL, "linear: %lld tiles", plan.tiles);
   // the staging loads address A and B rows with 32-bit byte offsets
   VK_UNSUPPORTED_IF(4LL * g.M * g.K >= (1LL << 32) || 4LL * g.N * g.Kp >= (1LL << 32),
                     "linear: operands of 4 GiB or more (M=%d, N=%d, K=%d)", g.M, g.N, g.K);
-  if (g.splits > 1) {
+  if (provided > 1) {
     VK_REQUIRE(g.N % 4 == 0, "linear: split-K needs out_features % 4 == 0");
-    const size_t need = static_cast<size_t>(g.splits) * g.M * g.N;
+    const size_t mn = static_cast<size_t>(g.M) * g.N;
     if (partial) {
-      VK_UNSUPPORTED_IF(need > partial_floats,
+      VK_UNSUPPORTED_IF(provided * mn > partial_floats,
                         "linear (M=%d, N=%d, K=%d): %d split-K slices need %zu floats of "
                         "scratch, more than the %zu available",
-                        g.M, g.N, g.K, g.splits, need, partial_floats);
+                        g.M, g.N, g.K, provided, provided * mn, partial_floats);
       g.partial = partial;
     } else {
-      VK_TRY(vk::ensure_work(rt, need, "linear (split-K)"));
+      const size_t most = provided > g.splits ? provided : g.splits;
+      VK_TRY(vk::ensure_work(rt, most * mn, "linear (split-K)"));
       g.partial = rt->work;
     }
   }

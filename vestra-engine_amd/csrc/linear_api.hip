@@ -173,6 +173,8 @@ LinearArgs linear_args(const vk_linear* lin, const vk_tensor* x, size_t rows, vk
   LinearArgs g{};
   g.x = static_cast<const float*>(x->ptr);
   g.wnk = lin->weight_nk;
+  g.wsplit = lin->weight_split;
+  g.wexp = lin->weight_exp;
   g.bias = lin->bias;
   g.ls = lin->ls_gamma;
   g.out = out ? static_cast<float*>(out->ptr) : nullptr;
@@ -205,6 +207,8 @@ int launch_linear(vk_runtime* rt, const vk_linear* lin, const vk_tensor* x, size
   LinearArgs g{};
   g.x = static_cast<const float*>(x->ptr);
   g.wnk = lin->weight_nk;
+  g.wsplit = lin->weight_split;
+  g.wexp = lin->weight_exp;
   g.bias = lin->bias;
   g.ls = lin->ls_gamma;
   g.out = static_cast<float*>(out->ptr);

@@ -1,0 +1,75 @@
+// F32 products on the f16 matrix cores.
+//
+// An f32 value is taken as two f16 values, x = x0 + x1 / 2^11: x0 is x rounded
+// to f16, x1 the remainder times 2^11 rounded to f16.  Two 11-bit significands
+// and the remainder's sign leave an error of at most 2^-23 |x| (rms about
+// 2^-25 |x|), with a floor of 2^-36 where x1 is a subnormal.  Of the four
+// products of two such values three are taken, in two f32 accumulators,
+//   main += x0 y0,   corr += x0 y1 + x1 y0,   sum = main + corr / 2^11;
+// the one left out is at most 2^-22 |x y| (rms about 2^-25).  The products are
+// exact, and main rounds once per 32 of k where the F32 matrix instruction
+// rounds once per 4: sums come out closer to the 64-bit values than from F32
+// products (K = 768: 1.4e-7 against 3.5-5.0e-7 relative), and
+// v_mfma_f32_16x16x32_f16 runs 16 times the F32 rate for three products.
+//
+// What the split cannot hold is found and computed from the f32 values:
+//  * |x| beyond f16's largest value, infinities and NaN: x0 is an infinity or
+//    a NaN, and so is every sum that x enters (is_finite below);
+//  * a row (the values of one sum) that is small as a whole, so that the floor
+//    counts: its largest |x| is below kRowMin and not 0.
+#pragma once
+
+#include "common.h"
+
+namespace vks {
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr float kUp = 2048.0f;          // 2^11
+constexpr float kDown = 1.0f / 2048.0f;
+// Rows whose largest value is at least this hold the 2^-36 floor below
+// sqrt(K) 2^-27 of that value.
+constexpr float kRowMin = 1.0f / 512.0f;
+
+// Both parts of two values, packed (a in the low half).
+__device__ __forceinline__ void split2(float a, float b, uint32_t* p0, uint32_t* p1) {
+  const f16x2 h = __builtin_convertvector((f32x2{a, b}), f16x2);
+  const f32x2 r = {__builtin_fmaf(static_cast<float>(h[0]), -kUp, a * kUp),
+                   __builtin_fmaf(static_cast<float>(h[1]), -kUp, b * kUp)};
+  *p0 = __builtin_bit_cast(uint32_t, h);
+  *p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2));
+}
+
+// Both parts of eight values, in the order of the values.
+__device__ __forceinline__ void split8(const float4& x, const float4& y, u32x4* p0, u32x4* p1) {
+  uint32_t h[4], l[4];
+  split2(x.x, x.y, &h[0], &l[0]);
+  split2(x.z, x.w, &h[1], &l[1]);
+  split2(y.x, y.y, &h[2], &l[2]);
+  split2(y.z, y.w, &h[3], &l[3]);
+  *p0 = u32x4{h[0], h[1], h[2], h[3]};
+  *p1 = u32x4{l[0], l[1], l[2], l[3]};
+}
+
+// The largest |x| of eight values and m (NaN left out).
+__device__ __forceinline__ float max_abs8(float m, const float4& x, const float4& y) {
+  m = fmaxf(fmaxf(m, fabsf(x.x)), fabsf(x.y));
+  m = fmaxf(fmaxf(m, fabsf(x.z)), fabsf(x.w));
+  m = fmaxf(fmaxf(m, fabsf(y.x)), fabsf(y.y));
+  return fmaxf(fmaxf(m, fabsf(y.z)), fabsf(y.w));
+}
+
+__device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ bool is_finite(float v) {
+  return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u;
+}
+
+}  // namespace vks

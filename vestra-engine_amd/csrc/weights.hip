@@ -41,6 +41,7 @@ int make_linear(vk_runtime* rt, size_t in, size_t out, const std::vector<float>&
   lin->out_features = out;
   lin->k_pitch = (in + kKAlign - 1) / kKAlign * kKAlign;
   int s = alloc_copy(wnk.data(), lin->k_pitch * out, &lin->weight_nk);
+  if (s == VK_OK) s = vk::split_weights(lin);
   if (s == VK_OK) s = vk::prepare_patch_filter(rt, lin);
   if (s == VK_OK) s = alloc_copy(bias, out, &lin->bias);
   if (s == VK_OK && ls) s = alloc_copy(ls, out, &lin->ls_gamma);
@@ -63,10 +64,9 @@ int make_linear(vk_runtime* rt, size_t in, size_t out, const std::vector<float>&
 // resident [out, kp] f32 layout.  Both conversions are exact (an f16 widens
 // exactly; d*q of an f16 scale and an int8 needs at most 19 significant
 // bits), so the projections give the bits of the f32 preparation of the
-// same widened weights.  The matrix cores stay on the F32 path: keeping
-// F16 / Q8_0 resident and widening inside the GEMM would add conversion
-// work to every tile for no gain in time (the projections are MFMA-bound)
-// nor in fit (288 GB of HBM).
+// same widened weights.
+// (The wide linear reads none of these f32 rows in its ordinary path: its
+// f16 parts are split from them once, when the linear is prepared.)
 // ---------------------------------------------------------------------------
 enum WeightSrc { kSrcF16 = 0, kSrcQ8 = 1 };
 constexpr int kQ8Block = 32;       // values per Q8_0 block (q8_0.rs:10)
@@ -150,6 +150,7 @@ int make_linear_stored(vk_runtime* rt, size_t in, size_t out, int src_kind, bool
     if (s == VK_OK && se != hipSuccess) s = vk::hip_fail(se, "hipStreamSynchronize");
     (void)hipFree(raw);
   }
+  if (s == VK_OK) s = vk::split_weights(lin);
   if (s == VK_OK) s = alloc_copy(bias, out, &lin->bias);
   if (s == VK_OK && ls) s = alloc_copy(ls, out, &lin->ls_gamma);
   if (s != VK_OK) {
@@ -276,6 +277,7 @@ int vk_linear_destroy(vk_linear* lin) {
   if (rt) (void)vk::bind_device(rt);
   if (rt) (void)hipStreamSynchronize(rt->stream);
   if (lin->weight_nk) (void)hipFree(lin->weight_nk);
+  if (lin->weight_split) (void)hipFree(lin->weight_split);
   if (lin->weight_patch) (void)hipFree(lin->weight_patch);
   if (lin->bias) (void)hipFree(lin->bias);
   if (lin->ls_gamma) (void)hipFree(lin->ls_gamma);
