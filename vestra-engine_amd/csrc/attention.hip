@@ -3,58 +3,73 @@
 // [n, 64] (a head of one view for local layers, a head of the whole flattened
 // multi-view sequence for global layers), with an online (one-pass) softmax.
 //
-// A 256-thread workgroup (4 waves) owns 64 queries of one sequence; wave w
-// owns queries 16w..16w+15 (unsplit launches over short sequences: 512
-// threads, 8 waves, 128 queries).  Grids of fewer than two 64-query
-// workgroups per CU (a single image's layer: 12 heads x 14 tiles) split
-// each tile's key blocks over several workgroups and merge the partial
-// results in a second pass (attention_kernel<true, 4>,
-// attention_merge_kernel).  Keys and values stream through LDS in blocks
-// of 64: K as [key][d] rows, V transposed as
-// [d][key] rows, both with a pitch of 68 floats (4 x odd: 16-row fragment
-// reads are bank-conflict free).
+// Both products run on the f16 matrix cores as three products of two-part
+// splits (split_f16.h), scaled so that the remainders stay normal numbers:
+// one accumulator, the small products first.
 //
-// Per key block a wave runs 128 v_mfma_f32_16x16x4_f32:
+// A workgroup of eight waves (or four, choose_plan) owns 32 queries a wave of
+// one sequence.  Grids of few tiles split the key blocks of each tile over
+// several workgroups and merge the partial results in a second pass
+// (attention_kernel<true, *>, attention_merge_kernel).  Keys and values stream
+// through LDS in blocks of 64 as f16 parts, split once per workgroup by the
+// thread that loaded them: K as [key][part][d] rows, V transposed as
+// [d][part][key] rows, both with a pitch of 272 bytes (16 x odd: fragment
+// reads of consecutive rows are bank-conflict free).  Two buffers, loads a
+// block ahead in registers, one barrier a block.
+//
+// Per key block a wave runs 48 v_mfma_f32_32x32x16_f16:
 //  * S^T = K Q^T (A = K, B = Q^T).  The transposed product leaves, in lane l,
-//    the scores of query l%16 for keys 16t + 4(l/16) + r (r = 0..3) of key
-//    tile t; the row max and sum of a query are then in-register over r and
-//    t plus two cross-group shuffles.
-//  * O += P V (A = P, B = V).  In the k-permuted fragment order used
-//    throughout this library (lane group g holds k = 16b + 4g + j in
-//    component j, MFMA step j takes component j) the A operand of key tile t
-//    is exactly the lane's four probabilities of that tile: P never leaves
-//    registers.  O's rows are queries 4(l/16) + r, so the per-query rescale
-//    factors reach them with four shuffles.
-// Scores are kept in the base-2 domain: Q is read once per workgroup and
-// pre-scaled by log2(e)/sqrt(64), so every softmax weight is one v_exp_f32
-// (2^x) of a difference of scores: p = 2^(s' - m') = e^(s - m).
+//    the scores of query l%32 for keys 32t + 8(r/4) + 4(l/32) + r%4 of key
+//    tile t; the row max and sum of a query are in-register plus one exchange
+//    with lane l ^ 32.
+//  * O^T += V^T P^T (A = V^T, B = P^T).  Key slots of a 16-key chunk are
+//    numbered so that lane l's eight slots are the eight keys whose weights it
+//    already holds: P never leaves registers, and V^T is stored in that order.
+//    O^T's columns are the lane's own query: rescales and the final division
+//    need no exchange.
+// Scores are kept in the base-2 domain: Q is pre-scaled by log2(e)/sqrt(64), so
+// every softmax weight is one v_exp_f32 (2^x) of an FMA of the score.  The
+// running maximum is only moved when a score passes it by more than 2^kSlack;
+// the weights carry 2^kPBits so that small ones keep both parts.
 // Keys past n are masked to -inf (last block only); queries past n are
 // computed on a clamped row and not stored.
 //
-// Staging: K goes to LDS row-major with 128-bit stores (16 lanes fill one
-// 256-byte key row).  V is transposed on the way in; its loads are mapped so
-// that the 64 lanes of a wave hold 16 keys x 4 float4 columns, which makes
-// every transposed 32-bit store of the wave hit 64 distinct banks.
+// What bounds it: per block and wave 1,536 cycles of MFMA against about 1,300
+// of VALU (32 weights a lane: FMA, exp, sum, split; the staging's conversions)
+// and, per CU, 2 x 34 KiB of fragment reads a wave pair from LDS.  12 x 10,392
+// rows: 920 us, 361 TFLOP/s of the product's own FLOP = 1,082 of f16 MFMA, 87%
+// of what a large f16 library product reaches on the card; with F32 matrix
+// instructions 2,478 us.  128-query workgroups there stage twice as often:
+// 1,064 us.
+//
+// Workgroups whose values the split cannot hold (a result that is not finite,
+// or values of V that are all tiny) compute their queries again with F32
+// matrix instructions (attention_tile_f32).
 #include <cmath>
 
 #include "common.h"
+#include "split_f16.h"
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+using vks::f32x16;
+using vks::f32x4;
+using vks::u32x4;
 
 constexpr int HD = 64;
 constexpr int KB = 64;  // keys per block
 constexpr int PITCH = 68;
 constexpr int kSlots = KB * HD / 4;  // float4 of one K (or V) block: 1024
 constexpr float kQScale = 0.125f * 1.44269504088896341f;  // log2(e) / sqrt(64)
-// Unsplit launches over sequences of at most this many rows run 128-query
-// workgroups of eight waves (two to a CU: four waves per SIMD, as four-wave
-// workgroups four to a CU give, with half the K/V staging per query): a
-// 12-view local layer (144 x 866) 259.6-265.4 -> 252.8-258.1 us, bits
-// unchanged.  The global layer (10,392 rows) measured 1% slower in
-// that form when it ran unsplit.
-constexpr int kWideTileMaxN = 1024;
+// Scales of the f16 parts (powers of two): K and V by 2^8, Q (with kQScale)
+// by 2^10, the weights by 2^11 with room for a factor 2^4 above the running
+// max.  |k|, |v| of 256 and |q| of 354 no longer fit (those tiles run in F32).
+constexpr float kKvUp = 256.0f, kQUp = 1024.0f, kSDown = 1.0f / 262144.0f;
+constexpr float kPBits = 11.0f, kPDown = 1.0f / 2048.0f, kSlack = 4.0f;
+constexpr float kODown = kPDown / kKvUp;
+constexpr int kFlush = 8;       // blocks between additions to the running total
+constexpr int kRowBytes = 272;  // LDS pitch of 64 values: 2 parts x 128 bytes + 16
+constexpr int kBufBytes = 2 * KB * kRowBytes;  // a block of K and of V
 static_assert(PITCH % 4 == 0 && (PITCH / 4) % 2 == 1, "pitch 4 x odd");
 static_assert(PITCH % 16 == 4, "transposed V stores: 16 (l >> 4) + (l & 15) covers 64 banks");
 
@@ -94,24 +109,29 @@ __device__ __forceinline__ float group_sum(float v) {
   return v + o;
 }
 
-// QG query groups of 16 (one wave each) per workgroup: 16 QG queries over
-// every key block.  PART: grids of fewer than two workgroups per CU (a
-// single image's layer: 12 heads x 14 query tiles) split the key blocks of
-// each query tile into `splits` contiguous runs, one workgroup each; a run
-// writes its O (scaled to its own running max), the max and the sum to
-// `part` ([splits][rows][64], then [splits][rows][2]) and
-// attention_merge_kernel combines them in split order.
-template <bool PART, int QG>
-__global__ __launch_bounds__(64 * QG) void attention_kernel(const float* __restrict__ q,
-                                                        const float* __restrict__ k,
-                                                        const float* __restrict__ v,
-                                                        float* __restrict__ out, int sequences,
-                                                        int n, int splits,
-                                                        float* __restrict__ part) {
-  constexpr int kThreads = 64 * QG;       // QG query groups (waves)
-  constexpr int QB = 16 * QG;             // queries per workgroup
-  constexpr int kPer = kSlots / kThreads; // staged float4 of K (and of V) per thread
-  __shared__ __align__(16) float smem[2 * KB * PITCH];
+__device__ __forceinline__ void split8_plain(const f32x4& x, const f32x4& y, u32x4* p0, u32x4* p1) {
+  uint32_t h[4], l[4];
+  vks::split2_plain(x[0], x[1], &h[0], &l[0]);
+  vks::split2_plain(x[2], x[3], &h[1], &l[1]);
+  vks::split2_plain(y[0], y[1], &h[2], &l[2]);
+  vks::split2_plain(y[2], y[3], &h[3], &l[3]);
+  *p0 = u32x4{h[0], h[1], h[2], h[3]};
+  *p1 = u32x4{l[0], l[1], l[2], l[3]};
+}
+
+// The same 64 queries with F32 matrix instructions (four waves of 16 queries;
+// a wave of an eight-wave workgroup past them only helps to stage), for
+// inputs that the split cannot hold.  In the k-permuted fragment order (lane
+// group g holds k = 16 b + 4 g + j in component j, MFMA step j takes component
+// j) the A operand of key tile t is the lane's four probabilities of that
+// tile; K is staged as [key][d] and V as [d][key] rows of 68 floats.
+template <bool PART, int kThreads>
+__device__ __forceinline__ void attention_tile_f32(
+    float* smem, const float* __restrict__ q, const float* __restrict__ k,
+    const float* __restrict__ v, float* __restrict__ out, int sequences, int n, int seq, int qb,
+    int kb_begin, int kb_end, int split, int splits, float* __restrict__ part) {
+  constexpr int kPer = kSlots / kThreads;  // staged float4 of K (and of V) per thread
+  constexpr int QG = kThreads / 64;
 
   const int tid = threadIdx.x;
   __builtin_assume(tid < kThreads);
@@ -120,13 +140,8 @@ __global__ __launch_bounds__(64 * QG) void attention_kernel(const float* __restr
   const int g = lane >> 4, c16 = lane & 15;
   float* Ks = smem;
   float* Vt = Ks + KB * PITCH;
-  const int nqb = (n + QB - 1) / QB;
-  // XCD-major numbering: the query blocks of one sequence share an XCD's L2
-  const int tile_all = vkd::xcd_tile(blockIdx.x, gridDim.x);
-  const int split = PART ? tile_all % splits : 0;
-  const int tile = PART ? tile_all / splits : tile_all;
-  const int seq = tile / nqb, q0 = (tile % nqb) * QB + wq * 16;
-  const bool live = q0 < n;  // uniform over the wave
+  const int q0 = qb + wq * 16;
+  const bool live = wq < 4 && q0 < n;  // uniform over the wave
   const size_t base = static_cast<size_t>(seq) * n * HD;
 
   // Q^T fragments (B operand): query q0 + c16, d = 16 bd + 4 g + j
@@ -169,9 +184,6 @@ __global__ __launch_bounds__(64 * QG) void attention_kernel(const float* __restr
                                           4 * ((lane >> 4) + 4 * (w2 >> 2)));
   }
 
-  const int nkb = (n + KB - 1) / KB;
-  const int kb_begin = PART ? split * nkb / splits : 0;
-  const int kb_end = PART ? (split + 1) * nkb / splits : nkb;
   for (int kb = kb_begin; kb < kb_end; ++kb) {
     const int k0 = kb * KB;
     f32x4 kr[kPer], vr[kPer];
@@ -295,6 +307,7 @@ __global__ __launch_bounds__(64 * QG) void attention_kernel(const float* __restr
     }
   }
 
+  if (!live) return;
   if constexpr (PART) {
     // this split's O (rescaled to its own running max), max and sum
     const size_t rows = static_cast<size_t>(sequences) * n;
@@ -326,6 +339,335 @@ __global__ __launch_bounds__(64 * QG) void attention_kernel(const float* __restr
       for (int dt = 0; dt < 4; ++dt) orow[16 * dt] = o[dt][r] / lr;
     }
   }
+}
+
+
+// A workgroup of QW waves, 32 queries each, over every key block.  PART: the
+// key blocks of each query tile are split into `splits` contiguous runs, one
+// workgroup each; a run writes its O (scaled to its own running max), the max
+// and the sum to `part` ([splits][rows][64], then [splits][rows][2]) and
+// attention_merge_kernel combines them in split order.
+template <bool PART, int QW>
+__global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __restrict__ q,
+                                                               const float* __restrict__ k,
+                                                               const float* __restrict__ v,
+                                                               float* __restrict__ out,
+                                                               int sequences, int n, int splits,
+                                                               float* __restrict__ part) {
+  constexpr int kThreads = 64 * QW;
+  constexpr int QB = 32 * QW;  // queries per workgroup
+  static_assert(QW == 4 || QW == 8, "four or eight waves");
+  // with eight waves the first four stage V and the others K
+  constexpr bool kShared = QW == 8;
+  __shared__ __align__(16) char smem[2 * kBufBytes];
+  __shared__ int flags[QW];
+
+  const int tid = threadIdx.x;
+  __builtin_assume(tid < kThreads);
+  const int wave = tid >> 6, lane = tid & 63;
+  const int half = lane >> 5, c32 = lane & 31;
+  const int nqb = (n + QB - 1) / QB;
+  // XCD-major numbering: the query blocks of one sequence share an XCD's L2
+  const int tile_all = vkd::xcd_tile(blockIdx.x, gridDim.x);
+  const int split = PART ? tile_all % splits : 0;
+  const int tile = PART ? tile_all / splits : tile_all;
+  const int seq = tile / nqb, qb = (tile % nqb) * QB;
+  const int q0 = qb + 32 * wave;
+  const bool live = q0 < n;  // uniform over the wave
+  const size_t base = static_cast<size_t>(seq) * n * HD;
+  const int nkb = (n + KB - 1) / KB;
+  const int kb_begin = PART ? static_cast<int>(static_cast<long long>(split) * nkb / splits) : 0;
+  const int kb_end =
+      PART ? static_cast<int>(static_cast<long long>(split + 1) * nkb / splits) : nkb;
+
+  // O^T: d = 32 dt + 8 (r / 4) + 4 half + r % 4 of query q0 + c32.  Blocks add
+  // to `o`, which moves to `total` every kFlush of them: a value is rounded 12
+  // times a block at the size of a few blocks, and then once per kFlush at
+  // that of the whole sum.
+  f32x16 o[2], total[2];
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[dt][r] = total[dt][r] = 0.0f;
+  float m_run = -INFINITY;  // running max of query q0 + c32 (both halves alike)
+  float l_run = 0.0f;       // sum over the keys that this lane holds
+  float vmax = 0.0f;        // largest |v| staged by this thread
+
+  // Staging, one block ahead through registers.  K: piece s = 8 floats, key
+  // s / 8, d 8 (s % 8).. ; V: 4 keys x 4 d per thread (its lanes in key order:
+  // a transposed 8-byte store of 16 lanes fills one 128-byte row).  Keys past
+  // n read past the sequence's buffer, which gives zeros (the block's offset
+  // is part of the lane's: the uniform offset is left out of bounds checks).
+  const int st = kShared ? tid & 255 : tid;
+  const bool upper = kShared && __builtin_amdgcn_readfirstlane(wave) >= 4;
+  const uint32_t bytes = 4u * static_cast<uint32_t>(n) * HD;
+  const int quad = st & 15, d4 = st >> 4;
+  // byte offsets of piece st, float4 i, in a block of K and of V
+  auto k_off = [&](int i) {
+    return 4u * static_cast<uint32_t>(((st >> 3) + 32 * (i >> 1)) * HD + 8 * (st & 7) + 4 * (i & 1));
+  };
+  auto v_off = [&](int i) { return 4u * static_cast<uint32_t>((4 * quad + i) * HD + 4 * d4); };
+  const __amdgpu_buffer_rsrc_t rsrc0 = vkd::buffer_rsrc((upper ? k : v) + base, bytes);
+  const __amdgpu_buffer_rsrc_t rsrc1 = vkd::buffer_rsrc(k + base, bytes);
+  uint32_t off0[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) off0[i] = upper ? k_off(i) : v_off(i);
+  float4 r0[4], r1[4];  // V (the upper waves: K), and K where a thread stages both
+  auto load_block = [&](int kb) {
+    const uint32_t blk = static_cast<uint32_t>(kb) * KB * HD * 4u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r0[i] = vkd::buffer_load4(rsrc0, blk + off0[i], 0);
+    if constexpr (!kShared) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r1[i] = vkd::buffer_load4(rsrc1, blk + k_off(i), 0);
+    }
+  };
+  load_block(kb_begin);
+
+  // Q^T fragments (B operand): query q0 + c32, d = 16 ks + 8 half + j
+  u32x4 qf[4][2];
+  {
+    const int qi = q0 + c32 < n ? q0 + c32 : n - 1;
+    const float* qrow = q + base + static_cast<size_t>(qi) * HD + 8 * half;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * ks) * kQScale * kQUp;
+      const f32x4 b = *reinterpret_cast<const f32x4*>(qrow + 16 * ks + 4) * kQScale * kQUp;
+      split8_plain(a, b, &qf[ks][0], &qf[ks][1]);
+    }
+  }
+
+  char* k_dst = smem + (st >> 3) * kRowBytes + 16 * (st & 7);
+  // V^T row d: [part][4 chunks of 16 keys], quad order 0 2 1 3 in a chunk
+  char* v_dst = smem + KB * kRowBytes + 4 * d4 * kRowBytes + 32 * (quad >> 2) +
+                16 * (quad & 1) + 8 * ((quad >> 1) & 1);
+  auto store_k = [&](int buf, const float4 (&kr)[4]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float4 x = kr[2 * i], y = kr[2 * i + 1];
+      u32x4 p0, p1;
+      split8_plain(f32x4{x.x, x.y, x.z, x.w} * kKvUp, f32x4{y.x, y.y, y.z, y.w} * kKvUp, &p0, &p1);
+      char* d = k_dst + buf * kBufBytes + 32 * i * kRowBytes;
+      *reinterpret_cast<u32x4*>(d) = p0;
+      *reinterpret_cast<u32x4*>(d + 128) = p1;
+    }
+  };
+  auto store_v4 = [&](char* d, float a, float b, float e, float f) {
+    uint32_t p0[2], p1[2];
+    vks::split2_plain(a * kKvUp, b * kKvUp, &p0[0], &p1[0]);
+    vks::split2_plain(e * kKvUp, f * kKvUp, &p0[1], &p1[1]);
+    *reinterpret_cast<uint2*>(d) = make_uint2(p0[0], p0[1]);
+    *reinterpret_cast<uint2*>(d + 128) = make_uint2(p1[0], p1[1]);
+  };
+  auto store_v = [&](int buf, const float4 (&vr)[4]) {
+    vmax = vks::max_abs8(vmax, vr[0], vr[1]);
+    vmax = vks::max_abs8(vmax, vr[2], vr[3]);
+    char* d = v_dst + buf * kBufBytes;
+    store_v4(d, vr[0].x, vr[1].x, vr[2].x, vr[3].x);
+    store_v4(d + kRowBytes, vr[0].y, vr[1].y, vr[2].y, vr[3].y);
+    store_v4(d + 2 * kRowBytes, vr[0].z, vr[1].z, vr[2].z, vr[3].z);
+    store_v4(d + 3 * kRowBytes, vr[0].w, vr[1].w, vr[2].w, vr[3].w);
+  };
+  auto store_block = [&](int buf) {
+    if (upper) {
+      store_k(buf, r0);
+    } else {
+      store_v(buf, r0);
+      if constexpr (!kShared) store_k(buf, r1);
+    }
+  };
+
+  const char* kfrag = smem + c32 * kRowBytes + 16 * half;
+  const char* vfrag = kfrag + KB * kRowBytes;
+  auto compute = [&](int kb, int buf) {
+    // S^T: s[t][r] = score of query q0 + c32 with key 32 t + 8 (r / 4) +
+    // 4 half + r % 4 of the block; small products first
+    f32x16 s[2];
+    u32x4 k0f[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+    const char* kf = kfrag + buf * kBufBytes;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const char* f = kf + 32 * t * kRowBytes + 32 * ks;
+        k0f[t][ks] = *reinterpret_cast<const u32x4*>(f);
+        const u32x4 k1 = *reinterpret_cast<const u32x4*>(f + 128);
+        s[t] = vks::mfma32(k1, qf[ks][0], s[t]);
+        s[t] = vks::mfma32(k0f[t][ks], qf[ks][1], s[t]);
+      }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) s[t] = vks::mfma32(k0f[t][ks], qf[ks][0], s[t]);
+    const int left = n - kb * KB;
+    if (left < KB) {  // the last, partial block
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (32 * t + 8 * (r / 4) + 4 * half + r % 4 >= left) s[t][r] = -INFINITY;
+    }
+    float mb = s[0][0];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mb = fmaxf(mb, s[t][r]);
+    mb *= kSDown;
+    // The running max follows only where a score passes it by more than
+    // kSlack (the weights keep that much room below f16's largest value).
+    if (__builtin_amdgcn_ballot_w64(mb > m_run + kSlack) != 0) {
+      float other;
+      mb = xor32_pair(mb, &other);
+      const float m_new = fmaxf(m_run, fmaxf(mb, other));
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 on the first block
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          o[dt][r] *= alpha;
+          total[dt][r] *= alpha;
+        }
+      l_run *= alpha;
+      m_run = m_new;
+    }
+    const float c = kPBits - m_run;
+    float ps = 0.0f;  // this block's weights (one addition to l_run a block)
+    const char* vf = vfrag + buf * kBufBytes;
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) {
+      const int t = ch >> 1, r0 = 8 * (ch & 1);
+      u32x4 vv[2][2];
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          vv[dt][p] = *reinterpret_cast<const u32x4*>(vf + 32 * dt * kRowBytes + 128 * p + 32 * ch);
+      u32x4 p0, p1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r0 + 2 * j], kSDown, c));
+        const float b = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r0 + 2 * j + 1], kSDown, c));
+        ps += a;
+        ps += b;
+        uint32_t x, y;
+        vks::split2_plain(a, b, &x, &y);
+        p0[j] = x;
+        p1[j] = y;
+      }
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) o[dt] = vks::mfma32(vv[dt][1], p0, o[dt]);
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) o[dt] = vks::mfma32(vv[dt][0], p1, o[dt]);
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) o[dt] = vks::mfma32(vv[dt][0], p0, o[dt]);
+    }
+    l_run += ps;
+  };
+
+  auto flush = [&]() {
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        total[dt][r] += o[dt][r];
+        o[dt][r] = 0.0f;
+      }
+  };
+  store_block(0);
+  __syncthreads();
+  for (int kb = kb_begin; kb < kb_end; ++kb) {
+    const int buf = (kb - kb_begin) & 1;
+    const bool more = kb + 1 < kb_end;
+    if (more) load_block(kb + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (live) {
+      if ((kb - kb_begin) % kFlush == kFlush - 1) flush();
+      compute(kb, buf);
+    }
+    if (more) store_block(buf ^ 1);
+    __syncthreads();
+  }
+
+  flush();
+
+  // Did the split hold everything?  (Any value of Q, K or V beyond f16, an
+  // infinity or a NaN makes the sums that it enters NaN or infinite.)
+  {
+    float other;
+    const float mine = xor32_pair(l_run, &other);
+    l_run = mine + other;
+  }
+  bool odd = live && !vks::is_finite(l_run);
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) odd |= live && !vks::is_finite(total[dt][r]);
+  // V is judged by the largest value of the run: two bits a wave
+  const bool big = vmax >= vks::kRowMin, some = vmax != 0.0f;
+  const int bits = (__builtin_amdgcn_ballot_w64(odd) ? 1 : 0) |
+                   (__builtin_amdgcn_ballot_w64(big) ? 2 : 0) |
+                   (__builtin_amdgcn_ballot_w64(some) ? 4 : 0);
+  if (lane == 0) flags[wave] = bits;
+  __syncthreads();
+  int all = 0;
+#pragma unroll
+  for (int w = 0; w < QW; ++w) all |= flags[w];
+  if (__builtin_expect((all & 1) || (all & 6) == 4, 0)) {
+#pragma unroll 1
+    for (int h = 0; h < QB / 64; ++h) {
+      __syncthreads();
+      attention_tile_f32<PART, kThreads>(reinterpret_cast<float*>(smem), q, k, v, out, sequences,
+                                         n, seq, qb + 64 * h, kb_begin, kb_end, split, splits,
+                                         part);
+    }
+    return;
+  }
+  const int qi = q0 + c32;
+  if (!live || qi >= n) return;
+  if constexpr (PART) {
+    // this split's O (rescaled to its own running max), max and sum
+    const size_t rows = static_cast<size_t>(sequences) * n;
+    const size_t row = static_cast<size_t>(split) * rows + static_cast<size_t>(seq) * n + qi;
+    float* po = part + row * HD + 4 * half;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<f32x4*>(po + 32 * dt + 8 * r) =
+            f32x4{total[dt][4 * r], total[dt][4 * r + 1], total[dt][4 * r + 2], total[dt][4 * r + 3]} * kODown;
+    if (half == 0)
+      *reinterpret_cast<float2*>(part + static_cast<size_t>(splits) * rows * HD + 2 * row) =
+          make_float2(m_run, l_run * kPDown);
+  } else {
+    // out[query][d] = O / l; both carry the weights' scale, O also V's
+    float* orow = out + base + static_cast<size_t>(qi) * HD + 4 * half;
+    const float l = l_run * kKvUp;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<f32x4*>(orow + 32 * dt + 8 * r) =
+            f32x4{total[dt][4 * r] / l, total[dt][4 * r + 1] / l, total[dt][4 * r + 2] / l,
+                  total[dt][4 * r + 3] / l};
+  }
+}
+
+// Sequences of at most one key block: a workgroup per sequence with F32
+// matrix instructions.  There is one short chain of loads, products and
+// stores, and nothing for the split to save: 12 x 38 5.5 us, 192 x 60 6.2 (the
+// kernel above: 6.1 and 6.8; from 65 rows on it is the faster, 8.1 to 11.7).
+__global__ __launch_bounds__(256) void attention_short_kernel(const float* __restrict__ q,
+                                                              const float* __restrict__ k,
+                                                              const float* __restrict__ v,
+                                                              float* __restrict__ out,
+                                                              int sequences, int n) {
+  __shared__ __align__(16) float smem[2 * KB * PITCH];
+  attention_tile_f32<false, 256>(smem, q, k, v, out, sequences, n, blockIdx.x, 0, 0, 1, 0, 1,
+                                 nullptr);
 }
 
 // Combines the key splits of the PART form: 16 threads per query row, one
@@ -364,6 +706,81 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __res
       f32x4{o[0] / l, o[1] / l, o[2] / l, o[3] / l};
 }
 
+// Key splits a caller must be ready to provide for: 1 where the shape never
+// splits (it can be captured before any eager call of its kind).  This is the
+// interface's rule, fixed apart from the splits that are taken: 64-query
+// tiles of fewer than two
+// workgroups per CU split to about two (at least two key blocks each, at most
+// 8); fuller grids where a model of 2.2 us per key block of the busiest CU,
+// the partial results' traffic at 5.5 TB/s and 3 us for the merge pass puts a
+// split at least 1% below the unsplit launch.
+int key_splits_to_provide(int cus, size_t sequences, size_t n) {
+  const long long tiles64 = static_cast<long long>(sequences) * ((n + 63) / 64);
+  const int nkb = static_cast<int>((n + KB - 1) / KB);
+  int splits = 1;
+  if (tiles64 < 2LL * cus) {
+    splits = static_cast<int>((2.0 * cus) / static_cast<double>(tiles64) + 0.5);
+    if (splits > nkb / 2) splits = nkb / 2;
+    if (splits > 8) splits = 8;
+    if (splits < 1) splits = 1;
+  } else {
+    constexpr double kBlockUs = 2.2, kBytesPerUs = 5.5e6, kMergeUs = 3.0;
+    const double row_bytes = 4.0 * (HD + 2) * static_cast<double>(sequences * n);
+    const double unsplit = kBlockUs * static_cast<double>((tiles64 + cus - 1) / cus * nkb);
+    double best = unsplit;
+    for (int sp = 2; sp <= 8 && 2 * sp <= nkb; ++sp) {
+      const long long load = (tiles64 * sp + cus - 1) / cus * ((nkb + sp - 1) / sp);
+      const double us = kBlockUs * static_cast<double>(load) +
+                        2.0 * sp * row_bytes / kBytesPerUs + kMergeUs;
+      if (us < best && us < 0.99 * unsplit) {
+        best = us;
+        splits = sp;
+      }
+    }
+  }
+  return splits;
+}
+
+// Waves per workgroup (eight: 256 queries, one workgroup a CU, half the K and V
+// staging per query; four: 128 queries, two a CU) and key splits, from a cost
+// model fitted to sweeps of 12 to 192 sequences of 256 to 10,392 rows: the
+// busiest CU runs ceil(tiles * s / CUs) workgroups of ceil(key blocks / s)
+// blocks each, 2.7 us per block of an eight-wave workgroup, 1.65 of a
+// four-wave one (2.0 where the CU has no second); a split adds its partial
+// results' traffic (s slices of rows x 66 floats written and read back at 5.5
+// TB/s) and the merge pass (about 3 us).  Measured (choice; neighbours): 12 x
+// 10,392 eight waves unsplit 920 us (2 splits 946, four waves 1064); 16 x 3,458
+// eight waves unsplit 150 (2 splits 165, four waves 178); 144 x 866 four waves
+// 104 (eight 124); 12 x 866 four waves in 3 splits 22.1 (unsplit 34.5, eight
+// waves in 4 splits 25.0); 12 x 1,732 eight waves in 3 splits 43 (four waves
+// 47, 2 splits 47).
+struct Plan {
+  int waves, splits;
+};
+
+Plan choose_plan(int cus, size_t sequences, size_t n, int provided) {
+  constexpr double kBytesPerUs = 5.5e6, kMergeUs = 3.0;
+  constexpr double kEightUs = 2.7, kFourUs = 1.65, kFourAloneUs = 2.0;
+  const long long nkb = static_cast<long long>((n + KB - 1) / KB);
+  const double row_bytes = 4.0 * (HD + 2) * static_cast<double>(sequences * n);
+  Plan best{4, 1};
+  double best_us = 0.0;
+  for (const int w : {4, 8}) {
+    const long long tiles = static_cast<long long>(sequences * ((n + 32 * w - 1) / (32 * w)));
+    for (int sp = 1; sp == 1 || (provided > 1 && sp <= 8 && sp <= nkb); ++sp) {
+      const long long load = (tiles * sp + cus - 1) / cus, blocks = (nkb + sp - 1) / sp;
+      double us = static_cast<double>(load * blocks) *
+                  (w == 8 ? kEightUs : (load > 1 ? kFourUs : kFourAloneUs));
+      if (sp > 1) us += 2.0 * sp * row_bytes / kBytesPerUs + kMergeUs;
+      if (best_us == 0.0 || us < best_us) {
+        best = Plan{w, sp};
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
 int check_qkv(const vk_tensor* t, size_t len, const char* what) {
   VK_REQUIRE(t && t->dtype == VK_F32 && t->len == len, "attention: %s must be f32 [%zu] (holds %zu)",
              what, len, t ? t->len : 0);
@@ -396,58 +813,33 @@ int vk_attention_into_f32(vk_runtime* rt, const vk_tensor* q, const vk_tensor* k
                "attention: out overlaps an input");
   }
   if (len == 0) return VK_OK;
-  // 64-query tiles.  When they give fewer than two workgroups per CU (one
-  // ViT-B image: 168 tiles), each tile's key blocks are split over about two
-  // workgroups per CU (at least two key blocks per split) and a second pass
-  // merges the partial results.  Fuller grids split only where the last
-  // round of workgroups leaves CUs unevenly loaded and a cost model puts the
-  // split at least 1% below the unsplit launch: the busiest CU runs
-  // ceil(tiles * s / CUs) workgroups of up to ceil(key blocks / s) blocks
-  // (about 2.2 us per block of one of the four workgroups a CU holds), and a
-  // split adds its partial results' traffic (s slices of rows x 66 floats
-  // written and read back) and the merge pass (about 3 us).  ViT-L at 3,458
-  // rows (880 tiles of 55 blocks, 3.4 per CU): 2 splits (425 us; unsplit
-  // 464); the 12-view global layer (1,956 tiles of 163 blocks, model 1.6%
-  // below unsplit): 3 splits (2,486 us; unsplit 2,582, 4 splits 2,528); the
-  // 12-view local layers (14 blocks per tile) stay unsplit (260 us; 3
-  // splits 288).
   const int cus = rt->cu_count > 0 ? rt->cu_count : 256;
-  const long long tiles64 = static_cast<long long>(sequences) * ((n + 63) / 64);
   const int nkb = static_cast<int>((n + KB - 1) / KB);
-  int splits = 1;
-  if (tiles64 < 2LL * cus) {
-    splits = static_cast<int>((2.0 * cus) / static_cast<double>(tiles64) + 0.5);
-    if (splits > nkb / 2) splits = nkb / 2;
-    if (splits > 8) splits = 8;
-    if (splits < 1) splits = 1;
-  } else {
-    constexpr double kBlockUs = 2.2, kBytesPerUs = 5.5e6, kMergeUs = 3.0;
-    const double row_bytes = 4.0 * (HD + 2) * static_cast<double>(sequences * n);
-    const double unsplit = kBlockUs * static_cast<double>((tiles64 + cus - 1) / cus * nkb);
-    double best = unsplit;
-    for (int sp = 2; sp <= 8 && 2 * sp <= nkb; ++sp) {
-      const long long load = (tiles64 * sp + cus - 1) / cus * ((nkb + sp - 1) / sp);
-      const double us = kBlockUs * static_cast<double>(load) +
-                        2.0 * sp * row_bytes / kBytesPerUs + kMergeUs;
-      if (us < best && us < 0.99 * unsplit) {
-        best = us;
-        splits = sp;
-      }
-    }
-  }
-  const long long blocks = tiles64 * splits;
+  const int provided = key_splits_to_provide(cus, sequences, n);
+  const Plan plan = choose_plan(cus, sequences, n, provided);
+  const int splits = plan.splits, qw = plan.waves;
+  const long long tiles = static_cast<long long>(sequences) * ((n + 32 * qw - 1) / (32 * qw));
+  const long long blocks = tiles * splits;
   VK_UNSUPPORTED_IF(blocks > 0x7fffffffLL, "attention: %lld workgroups", blocks);
   const auto* Q = static_cast<const float*>(q->ptr);
   const auto* K = static_cast<const float*>(k->ptr);
   const auto* V = static_cast<const float*>(v->ptr);
   auto* O = static_cast<float*>(out->ptr);
   const int S = static_cast<int>(sequences), N = static_cast<int>(n);
+  if (provided > 1) {
+    const size_t rows = sequences * n;
+    const int most = provided > splits ? provided : splits;
+    VK_TRY(vk::ensure_work(rt, static_cast<size_t>(most) * rows * (HD + 2), "attention"));
+  }
   if (splits > 1) {
     const size_t rows = sequences * n;
-    VK_TRY(vk::ensure_work(rt, static_cast<size_t>(splits) * rows * (HD + 2), "attention"));
     float* part = rt->work;
-    hipLaunchKernelGGL((attention_kernel<true, 4>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(256), 0, rt->stream, Q, K, V, O, S, N, splits, part);
+    if (qw == 8)
+      hipLaunchKernelGGL((attention_kernel<true, 8>), dim3(static_cast<unsigned>(blocks)),
+                         dim3(512), 0, rt->stream, Q, K, V, O, S, N, splits, part);
+    else
+      hipLaunchKernelGGL((attention_kernel<true, 4>), dim3(static_cast<unsigned>(blocks)),
+                         dim3(256), 0, rt->stream, Q, K, V, O, S, N, splits, part);
     VK_TRY(vk::check_launch("attention_kernel"));
     const long long threads = static_cast<long long>(rows) * 16;
     const dim3 mgrid(static_cast<unsigned>((threads + 255) / 256));
@@ -465,16 +857,15 @@ int vk_attention_into_f32(vk_runtime* rt, const vk_tensor* q, const vk_tensor* k
     }
     return vk::check_launch("attention_merge_kernel");
   }
-  if (n <= kWideTileMaxN) {
-    // unsplit short sequences: 128-query workgroups (eight waves), half the
-    // K/V staging per query
-    const long long t128 = static_cast<long long>(sequences) * ((n + 127) / 128);
-    hipLaunchKernelGGL((attention_kernel<false, 8>), dim3(static_cast<unsigned>(t128)), dim3(512),
+  if (nkb == 1)
+    hipLaunchKernelGGL(attention_short_kernel, dim3(static_cast<unsigned>(sequences)), dim3(256), 0,
+                       rt->stream, Q, K, V, O, S, N);
+  else if (qw == 8)
+    hipLaunchKernelGGL((attention_kernel<false, 8>), dim3(static_cast<unsigned>(blocks)), dim3(512),
                        0, rt->stream, Q, K, V, O, S, N, 1, nullptr);
-    return vk::check_launch("attention_kernel");
-  }
-  hipLaunchKernelGGL((attention_kernel<false, 4>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                     rt->stream, Q, K, V, O, S, N, 1, nullptr);
+  else
+    hipLaunchKernelGGL((attention_kernel<false, 4>), dim3(static_cast<unsigned>(blocks)), dim3(256),
+                       0, rt->stream, Q, K, V, O, S, N, 1, nullptr);
   return vk::check_launch("attention_kernel");
 }
 

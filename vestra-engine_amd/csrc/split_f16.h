@@ -27,6 +27,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kUp = 2048.0f;          // 2^11
@@ -55,6 +56,16 @@ __device__ __forceinline__ void split8(const float4& x, const float4& y, u32x4* 
   *p1 = u32x4{l[0], l[1], l[2], l[3]};
 }
 
+// Both parts with the remainder left at its own scale, x = x0 + x1: for values
+// scaled up beforehand (the floor is 2^-25 of the scaled value), summed in one
+// accumulator.
+__device__ __forceinline__ void split2_plain(float a, float b, uint32_t* p0, uint32_t* p1) {
+  const f16x2 h = __builtin_convertvector((f32x2{a, b}), f16x2);
+  const f32x2 r = {a - static_cast<float>(h[0]), b - static_cast<float>(h[1])};
+  *p0 = __builtin_bit_cast(uint32_t, h);
+  *p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2));
+}
+
 // The largest |x| of eight values and m (NaN left out).
 __device__ __forceinline__ float max_abs8(float m, const float4& x, const float4& y) {
   m = fmaxf(fmaxf(m, fabsf(x.x)), fabsf(x.y));
@@ -65,6 +76,11 @@ __device__ __forceinline__ float max_abs8(float m, const float4& x, const float4
 
 __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
