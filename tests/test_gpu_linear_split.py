@@ -35,11 +35,11 @@ def _check(got, x, w, b, label):
     assert not bad.any(), f"{label}: {int(bad.sum())} off, worst {np.max(np.abs(got - ref) / tol)}"
 
 
-# tiles 64 x 64 (2 stages a barrier: odd counts, tails), 64 x 128, 128 x 128,
+# tiles 128 x 256 (10392 x 64 -> 768, 4000 x 1024 -> 1028), 64 x 64 (2 stages a barrier: odd counts, tails), 64 x 128, 128 x 128,
 # rows and columns one past a tile, split runs, K below one stage
 @pytest.mark.parametrize("m,k,n", [(1, 4, 4), (63, 28, 60), (65, 96, 68), (64, 100, 64),
                                    (130, 3072, 132), (1500, 160, 2304), (10392, 64, 768),
-                                   (4097, 132, 1540)])
+                                   (4097, 132, 1540), (4000, 1024, 1028)])
 def test_shapes(rt, rng, m, k, n):
     x, w, b = normals(rng, m, k), normals(rng, k, n, scale=0.02), normals(rng, n, scale=0.02)
     _check(_linear(rt, x, w, b), x, w, b, f"{m}x{k}->{n}")

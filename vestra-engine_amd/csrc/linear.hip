@@ -5,9 +5,9 @@
 // The products run on the f16 matrix cores as three products of two-part
 // splits (split_f16.h), F32 in, F32 accumulate.
 //
-// A 256-thread workgroup owns a TM x TN output tile (128 x 128; 64 x 128 or
-// 64 x 64 for grids of few rows); wave w computes all TM rows of columns
-// TN/4 w .. + TN/4 as TM/16 x TN/64 tiles of v_mfma_f32_16x16x32_f16.
+// A workgroup owns a TM x TN output tile (128 x 256 with eight waves, 128 x 128
+// with four; 64 x 128 or 64 x 64 for grids of few rows); a wave computes all TM
+// rows of 32 columns (64 x 64 tiles: 16) with v_mfma_f32_16x16x32_f16.
 //
 //  * A (activations, f32) is read by raw buffer loads one stage ahead, split
 //    by the thread that loaded it and staged through LDS as [row][part][32 k]
@@ -23,7 +23,14 @@
 //
 // A 128 x 128 tile runs 48 MFMAs a wave (768 cycles) per 32 k on 8 x 2
 // fragment reads from LDS (4 waves: 512 cycles of its 128 bytes a clock)
-// and 16 + 16 KiB from L2; two workgroups a CU cover each other's barriers.
+// and 16 + 16 KiB from L2; two workgroups a CU cover each other's barriers.  A
+// 128 x 256 tile splits and reads A once for twice the columns: 10,392 x 3072
+// -> 768 in 127 us against 136 (386 TFLOP/s of the product's FLOP, 1,160 of f16
+// MFMA; a large f16 library product reaches 1,243 on the card).  What bounds
+// both is the matrix pipe at the clock that its power allows (about 2.0 GHz,
+// 50% busy); bank conflicts of the staging stores do not show (a conflict-free
+// plane layout measured the same), lines of A touched more often do (a lane
+// per row instead of four: 10-20% slower).
 // Grids of few tiles split K over several workgroups per tile (split-K:
 // partial sums in the runtime's work buffer, added in split order by
 // splitk_reduce_kernel).
@@ -63,7 +70,8 @@ using vks::u32x4;
 
 constexpr int KC = vk::kSplitK;    // k of one stage (and of one MFMA)
 constexpr int kParts = 2;           // f16 parts of a weight
-constexpr int kThreads = 256;      // four waves
+// Waves of a tile: one per 32 columns, at least four.
+constexpr int waves_for(int tn) { return tn == 256 ? 8 : 4; }
 constexpr int kRowBytes = 144;     // LDS pitch of a row of A: 2 parts x 64 bytes + 16
 constexpr int kXsPitch = 68;       // f32 pitch of the Q/K epilogue's rows
 static_assert(kRowBytes % 16 == 0 && (kRowBytes / 16) % 2 == 1 && kRowBytes >= 4 * KC, "pitch");
@@ -194,10 +202,11 @@ __device__ __forceinline__ void tile_of(int t, int gmt, int gnt, int splits, int
 // KS: stages of 32 k per barrier (2 for the 64-row tiles, whose 12 or 24
 // MFMAs a wave and stage are too few to cover a load's latency).
 template <int EPI, int LAY, int QKN, int TM, int TN, int KS>
-__global__ __launch_bounds__(kThreads, 2) void linear_wide_kernel(LinearArgs g) {
+__global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(LinearArgs g) {
+  constexpr int kWaves = waves_for(TN), kThreads = 64 * kWaves;
   static_assert(TM == 128 || TM == 64, "tile heights 128 and 64");
-  static_assert(TN == 128 || TN == 64, "tile widths 128 and 64");
-  constexpr int WN = TN / 4;            // columns of a wave
+  static_assert(TN == 256 || TN == 128 || TN == 64, "tile widths 256, 128 and 64");
+  constexpr int WN = TN / kWaves;       // columns of a wave
   constexpr int MT = TM / 16;           // 16-row MFMA tiles of a wave
   constexpr int NU = WN / 16;           // 16-column MFMA tiles of a wave
   constexpr int kSlots = TM * 4 * KS;   // 8-k pieces of A a barrier
@@ -388,7 +397,10 @@ __global__ __launch_bounds__(kThreads, 2) void linear_wide_kernel(LinearArgs g) 
   const bool wave_odd = __builtin_amdgcn_ballot_w64(odd) != 0;
   if (lane == 0) flags[wave] = wave_odd;
   __syncthreads();
-  if (__builtin_expect(flags[0] | flags[1] | flags[2] | flags[3], 0)) {
+  int any = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) any |= flags[w];
+  if (__builtin_expect(any, 0)) {
     // The tile again, with F32 matrix instructions (fragment order: lane
     // group g4 holds k = 16 b + 4 g4 + j of block b in component j).
     constexpr int kPitchF = kRowBytes / 4;
@@ -454,9 +466,9 @@ __global__ __launch_bounds__(kThreads, 2) void linear_wide_kernel(LinearArgs g) 
   // loaded, on clamped indices, before the first store.
   if constexpr (QKN != 0) {
     static_assert(LAY == kQkvHnd && EPI == kLinStore, "Q/K epilogue of the QKV projection");
-    // A head of Q, K or V is two waves of a 128-wide tile or all four of a
-    // 64-wide one; its 64-row halves meet in LDS one after the other.
-    constexpr int kHeadWaves = 256 / TN;              // 2 or 4
+    // A head of Q, K or V is two waves' columns, or all four's of a 64-wide
+    // tile; its 64-row halves meet in LDS one after the other.
+    constexpr int kHeadWaves = 64 / WN;               // 2 or 4
     constexpr int kRowsPerGroup = 16 / kHeadWaves;    // rows of a 16-lane group a half
     const int head = wave / kHeadWaves, hw = wave % kHeadWaves;
     const int col0 = n0 + head * 64;
@@ -700,30 +712,36 @@ int slices_to_provide(long long cus, int M, int N, int K) {
 // Tile shape and split count, from a cost model fitted to plan sweeps of
 // the ViT-B and ViT-L projections at 100 to 10,392 rows.  Workgroups are
 // dealt round-robin to the CUs, so the busiest CU runs ceil(tiles * s / CUs)
-// workgroups of up to ceil(stages / s) 32-wide K stages each: 0.85 us per
-// stage of a 128 x 128 tile, 0.43 of a 64 x 128 and 0.26 of a 64 x 64 one (a
-// quarter of the MFMAs on half the operands); a CU with one workgroup has
-// nothing to cover its waits and counts 1.3.  A split adds its partial sums
-// (s x M x N floats written, then read by the sum pass, at about 5.5 TB/s)
-// and the sum pass's launch (about 2 us).  The cheapest plan wins; on ties
-// the larger tile, then the smaller count.  At least four stages per split;
-// where the shape may split, at most kMaxStages of them (a run's rounding
-// grows with its length: K = 4096, 4.1e-7 of the 64-bit result unsplit, 3.0e-7
-// in two).  Measured (model's choice; neighbours): 866 x 768 -> 2304, 64 x 64
-// 18.3 us (64 x 128 19.3, 128 x 128 28); 866 x 3072 -> 768, 64 x 64 x 3 24.7
-// (unsplit 35, 64 x 128 x 6 24.4); 1500 x 768 -> 2304, 64 x 128 26.0 (64 x 64
-// 29.6, 128 x 128 31.5); 10,392 x 3072 -> 768, 128 x 128 155 (64 x 128 161, 64
-// x 64 198).
+// workgroups of up to ceil(stages / s) 32-wide K stages each: 1.3 us per stage
+// of a 128 x 256 tile (and 3 us per tile that nothing else on the CU covers),
+// 0.85 of a 128 x 128, 0.43 of a 64 x 128 and 0.26 of a 64 x 64 one; of the
+// latter three, a CU with one workgroup has nothing to cover its waits and
+// counts 1.3.  A split adds its partial sums (s x M x N floats written, then
+// read by the sum pass, at about 5.5 TB/s) and the sum pass's launch (about 2
+// us).  The cheapest plan wins; on ties the first shape, then the smaller
+// count.  At least four stages per
+// split; where the shape may split, at most kMaxStages of them (a run's
+// rounding grows with its length: K = 4096, 4.1e-7 of the 64-bit result
+// unsplit, 3.0e-7 in two).  Measured (model's choice; neighbours): 866 x 768 ->
+// 2304, 64 x 64 17.2 us (64 x 128 18.2, 128 x 128 29); 866 x 3072 -> 768, 64 x
+// 64 x 3 24.4 (unsplit 35, 64 x 128 x 6 24.3); 1500 x 768 -> 2304, 64 x 128 24.3
+// (64 x 64 27, 128 x 128 30); 3458 x 4096 -> 1024, 128 x 256 x 2 90 (64 x 128
+// 97, 128 x 128 x 2 99); 10,392 x 3072 -> 768, 128 x 256 127 (128 x 128 136, 64
+// x 128 154).
 constexpr int kMaxStages = 96;
 
 Plan choose_plan(long long cus, int M, int N, int K, int provided) {
   constexpr double kBytesPerUs = 5.5e6, kSumLaunchUs = 2.0, kAlone = 1.3;
-  // tile shape, us of one of its K stages
+  // tile shape, us of one of its K stages, of one of its tiles, and the load
+  // that a lone workgroup counts
   struct Shape {
     int tm, tn;
-    double us;
+    double us, tile_us, alone;
   };
-  constexpr Shape kShapes[] = {{128, 128, 0.85}, {64, 128, 0.43}, {64, 64, 0.26}};
+  constexpr Shape kShapes[] = {{128, 256, 1.3, 3.0, 1.0},
+                               {128, 128, 0.85, 0.0, kAlone},
+                               {64, 128, 0.43, 0.0, kAlone},
+                               {64, 64, 0.26, 0.0, kAlone}};
   const int nch = (K + KC - 1) / KC;
   const long long mn = static_cast<long long>(M) * N;
   // the shortest run is kMaxStages or, if the slices do not allow that, 1 / max
@@ -739,7 +757,7 @@ Plan choose_plan(long long cus, int M, int N, int K, int provided) {
       const int stages = (nch + sp - 1) / sp;
       if (stages > kMaxStages && may(sp + 1)) continue;
       const double load = static_cast<double>((tiles * sp + cus - 1) / cus);
-      double us = sh.us * stages * (load > 1.0 ? load : kAlone);
+      double us = (sh.us * stages + sh.tile_us) * (load > 1.0 ? load : sh.alone);
       if (sp > 1) us += 8.0 * static_cast<double>(sp * mn) / kBytesPerUs + kSumLaunchUs;
       if (best.tm == 0 || us < best_us) {
         best = Plan{sh.tm, sh.tn, sp, tiles};
@@ -753,14 +771,17 @@ Plan choose_plan(long long cus, int M, int N, int K, int provided) {
 template <int EPI, int LAY, int QKN = 0>
 void launch_pair(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 grid,
                  bool sum_pass = true) {
-  if (plan.tm == 128)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 128, 1>), grid, dim3(kThreads), 0,
+  if (plan.tn == 256)
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 256, 1>), grid, dim3(512), 0,
+                       rt->stream, g);
+  else if (plan.tm == 128)
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 128, 1>), grid, dim3(256), 0,
                        rt->stream, g);
   else if (plan.tn == 128)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 128, 2>), grid, dim3(kThreads), 0,
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 128, 2>), grid, dim3(256), 0,
                        rt->stream, g);
   else
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 64, 2>), grid, dim3(kThreads), 0,
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 64, 2>), grid, dim3(256), 0,
                        rt->stream, g);
   if (g.splits > 1 && sum_pass) {
     const long long n4 = static_cast<long long>(g.M) * g.N / 4;
@@ -886,6 +907,7 @@ int launch_linear_wide(vk_runtime* rt, const LinearArgs& g0, int epi, float* par
       g.partial = rt->work;
     }
   }
+  VK_REQUIRE(g.splits == 1 || g.partial, "linear: a split plan without partial sums");
   const dim3 grid(static_cast<unsigned>(plan.tiles * g.splits));
   // LayerNorm after the residual epilogue: in the sum pass when there is
   // one and a row is 768 or 1024 floats, else as a separate pass
