@@ -26,11 +26,11 @@ def _linear(rt, x, w, b):
     return out.numpy().reshape(m, n)
 
 
-def _check(got, x, w, b, label):
+def _check(got, x, w, b, label, floor=0.0):
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     ref = x64 @ w64 + b
     tol = (2 * np.sqrt(x.shape[1]) * U * (np.abs(x64) @ np.abs(w64)) + U * np.abs(ref)
-           + U * np.abs(b) + 2.0 ** -149)
+           + U * np.abs(b) + 2.0 ** -149 + floor * np.abs(w64).sum(axis=0))
     bad = np.abs(got - ref) > tol
     assert not bad.any(), f"{label}: {int(bad.sum())} off, worst {np.max(np.abs(got - ref) / tol)}"
 
@@ -84,3 +84,25 @@ def test_infinities_and_nan_stay_in_their_rows_and_columns(rt, rng, m, k, n):
     rows = [r for r in range(m) if r not in (3, 4, m - 1)]
     cols = [c for c in range(n) if c not in (9, n - 1)]
     _check(got[np.ix_(rows, cols)], x[rows], w[:, cols], b[cols], "finite part")
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 96, 128), (130, 3072, 132), (1500, 768, 2304),
+                                   (5000, 64, 768), (4000, 1024, 1028)])
+@pytest.mark.parametrize("wide_range", [False, True])
+def test_f16_stored_weights_are_the_f32_preparation(rt, rng, m, k, n, wide_range):
+    """Weights stored as f16 take one part and two products, unless a column's
+    range needs the second part (f16's largest value beside subnormals): the
+    bits of the f32 preparation of the same values either way."""
+    x, b = normals(rng, m, k), normals(rng, n, scale=0.02)
+    w = normals(rng, k, n, scale=0.02).astype(np.float16)
+    if wide_range:
+        w[0, :] = 60000.0
+        w[1:3, :] = np.float16(2.0 ** -24) * 3
+        x[:, 0] *= np.float32(1e-6)
+    out = rt.alloc_f32(m * n)
+    rt.prepare_linear_w16(k, n, w, b).run_into(rt.upload_f32(x), m, out)
+    assert np.array_equal(out.numpy().reshape(m, n), _linear(rt, x, w.astype(np.float32), b))
+    # the split of x has a floor of 2^-36 of 1, which weights of 60000 against
+    # values of 1e-6 (where they give 0.06) make visible: 2^-36 sum_k |w_k|
+    _check(out.numpy().reshape(m, n), x, w.astype(np.float32), b, "f16 weights",
+           floor=2.0 ** -36 if wide_range else 0.0)

@@ -65,10 +65,11 @@ struct vk_linear {
   size_t out_features = 0;
   size_t k_pitch = 0;          // in_features rounded up to 16
   float* weight_nk = nullptr;  // [out, k_pitch], input dimension contiguous
-  // The rows as two f16 parts in the wide linear's fragment order, each row
+  // The rows as f16 parts in the wide linear's fragment order, each row
   // scaled by 2^weight_exp (split_weights), for in_features % 4 == 0.
   void* weight_split = nullptr;
   int* weight_exp = nullptr;   // [out], in weight_split's allocation
+  int weight_parts = 0;        // 1 where every second part is zero (f16 values)
   // For a 3x14x14 patch filter (in_features 588) only: the same rows with
   // the input dimension reordered (c, ky, kx) -> (ky, kx, c), the order in
   // which an HWC image holds a patch.
@@ -174,7 +175,8 @@ void noalloc_setup(int device);
 int prepare_patch_filter(vk_runtime* rt, vk_linear* lin);
 // Allocates and fills lin->weight_split and weight_exp from lin->weight_nk (whose writes have
 // finished); the default stream, waited for.  in_features % 4 != 0: nothing.
-int split_weights(vk_linear* lin);
+// f16_values: the weights were stored as f16.
+int split_weights(vk_linear* lin, bool f16_values);
 // Makes rt->work hold at least `floats` floats (at least 8 Mi once
 // allocated, doubling on growth).  Growth is refused during stream capture:
 // run the sequence once eagerly first.  The buffer it replaces is retired,
@@ -221,6 +223,7 @@ struct LinearArgs {
   const float* wnk;   // [N, Kp], K contiguous, zero beyond K
   const void* wsplit; // its f16 parts (vk_linear::weight_split) and
   const int* wexp;    // their rows' exponents, linear.hip only
+  int wparts;         // parts of a weight (vk_linear::weight_parts)
   const float* bias;  // [N]
   const float* ls;    // [N] or null
   float* out;         // [M, N]

@@ -69,7 +69,6 @@ using vks::f32x4;
 using vks::u32x4;
 
 constexpr int KC = vk::kSplitK;    // k of one stage (and of one MFMA)
-constexpr int kParts = 2;           // f16 parts of a weight
 // Waves of a tile: one per 32 columns, at least four.
 constexpr int waves_for(int tn) { return tn == 256 ? 8 : 4; }
 constexpr int kRowBytes = 144;     // LDS pitch of a row of A: 2 parts x 64 bytes + 16
@@ -199,9 +198,12 @@ __device__ __forceinline__ void tile_of(int t, int gmt, int gnt, int splits, int
   *split = rest / gnt;
 }
 
+// NP: f16 parts of a weight.  Weights that are f16 values have one (the other
+// is all zeros, so the sums are the same): two products, half of B's bytes.
+//
 // KS: stages of 32 k per barrier (2 for the 64-row tiles, whose 12 or 24
 // MFMAs a wave and stage are too few to cover a load's latency).
-template <int EPI, int LAY, int QKN, int TM, int TN, int KS>
+template <int EPI, int LAY, int QKN, int TM, int TN, int KS, int NP>
 __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(LinearArgs g) {
   constexpr int kWaves = waves_for(TN), kThreads = 64 * kWaves;
   static_assert(TM == 128 || TM == 64, "tile heights 128 and 64");
@@ -284,7 +286,7 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   };
 
   // B: 16-column tile j of the weights, stage ch, part p: 64 x 16 bytes at
-  // ((j nch + ch) 2 + p) KiB.  Tiles past N read the last one; their columns
+  // ((j nch + ch) NP + p) KiB.  Tiles past N read the last one; their columns
   // are not stored.
   const int ntiles = (g.N + 15) / 16;
   const u32x4* bptr[NU];
@@ -293,9 +295,9 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
     const int j = (n0 + wave * WN) / 16 + u;
     const int cj = j < ntiles ? j : ntiles - 1;
     bptr[u] = reinterpret_cast<const u32x4*>(g.wsplit) +
-              static_cast<size_t>(cj) * nch * (kParts * 64) + lane;
+              static_cast<size_t>(cj) * nch * (NP * 64) + lane;
   }
-  auto load_b = [&](int ch0, u32x4 (&b)[KS][NU][kParts]) {
+  auto load_b = [&](int ch0, u32x4 (&b)[KS][NU][NP]) {
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       // a stage past the split's end multiplies zeros of A
@@ -303,8 +305,8 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
 #pragma unroll
       for (int u = 0; u < NU; ++u)
 #pragma unroll
-        for (int p = 0; p < kParts; ++p)
-          b[s][u][p] = bptr[u][static_cast<size_t>(ch) * (kParts * 64) + p * 64];
+        for (int p = 0; p < NP; ++p)
+          b[s][u][p] = bptr[u][static_cast<size_t>(ch) * (NP * 64) + p * 64];
     }
   };
   const char* afrag = smem + (lane & 15) * kRowBytes + 16 * (lane >> 4);
@@ -314,7 +316,7 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
 #pragma unroll
     for (int u = 0; u < NU; ++u) acc[t][u] = corr[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
   // Fragments of the next 16 rows are read while these rows' MFMAs run.
-  auto mma = [&](int buf, const u32x4 (&b)[KS][NU][kParts]) {
+  auto mma = [&](int buf, const u32x4 (&b)[KS][NU][NP]) {
     u32x4 a[2][2];
     auto read_a = [&](int st, u32x4 (&f)[2]) {
       const char* ar = afrag + buf * kBufBytes + (st / MT) * kStageBytes +
@@ -331,8 +333,10 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
       const u32x4(&f)[2] = a[st & 1];
 #pragma unroll
       for (int u = 0; u < NU; ++u) acc[t][u] = vks::mfma(f[0], b[s][u][0], acc[t][u]);
+      if constexpr (NP == 2) {
 #pragma unroll
-      for (int u = 0; u < NU; ++u) corr[t][u] = vks::mfma(f[0], b[s][u][1], corr[t][u]);
+        for (int u = 0; u < NU; ++u) corr[t][u] = vks::mfma(f[0], b[s][u][NP - 1], corr[t][u]);
+      }
 #pragma unroll
       for (int u = 0; u < NU; ++u) corr[t][u] = vks::mfma(f[1], b[s][u][0], corr[t][u]);
       __builtin_amdgcn_sched_barrier(0);
@@ -342,7 +346,7 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   // One stage: split and store what was loaded a stage earlier, issue the
   // next stage's loads, run this one's MFMAs.  A buffer is written again two
   // stages after it was read, with a barrier in between.
-  u32x4 b0[KS][NU][kParts], b1[KS][NU][kParts];
+  u32x4 b0[KS][NU][NP], b1[KS][NU][NP];
   load_a(c_begin);
   load_b(c_begin, b0);
   int ch = c_begin;
@@ -768,21 +772,29 @@ Plan choose_plan(long long cus, int M, int N, int K, int provided) {
   return best;
 }
 
+template <int EPI, int LAY, int QKN, int NP>
+void launch_tiles(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 grid) {
+  if (plan.tn == 256)
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 256, 1, NP>), grid, dim3(512), 0,
+                       rt->stream, g);
+  else if (plan.tm == 128)
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 128, 1, NP>), grid, dim3(256), 0,
+                       rt->stream, g);
+  else if (plan.tn == 128)
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 128, 2, NP>), grid, dim3(256), 0,
+                       rt->stream, g);
+  else
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 64, 2, NP>), grid, dim3(256), 0,
+                       rt->stream, g);
+}
+
 template <int EPI, int LAY, int QKN = 0>
 void launch_pair(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 grid,
                  bool sum_pass = true) {
-  if (plan.tn == 256)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 256, 1>), grid, dim3(512), 0,
-                       rt->stream, g);
-  else if (plan.tm == 128)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 128, 1>), grid, dim3(256), 0,
-                       rt->stream, g);
-  else if (plan.tn == 128)
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 128, 2>), grid, dim3(256), 0,
-                       rt->stream, g);
+  if (g.wparts == 1)
+    launch_tiles<EPI, LAY, QKN, 1>(rt, g, plan, grid);
   else
-    hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 64, 64, 2>), grid, dim3(256), 0,
-                       rt->stream, g);
+    launch_tiles<EPI, LAY, QKN, 2>(rt, g, plan, grid);
   if (g.splits > 1 && sum_pass) {
     const long long n4 = static_cast<long long>(g.M) * g.N / 4;
     const dim3 sgrid(static_cast<unsigned>((n4 + 255) / 256));
@@ -811,6 +823,7 @@ void launch_pair(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 gri
 __global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __restrict__ wnk,
                                                               int* __restrict__ wexp, int N,
                                                               int Kp) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) wexp[N] = 0;  // split_weights_kernel's flag
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= N) return;
   uint32_t m = 0;
@@ -829,13 +842,15 @@ __global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __res
 }
 
 // The f16 parts of the scaled rows 2^wexp[n] wnk[n] of [N, Kp] in the order
-// the wide kernel's lanes read them: 16-row tile j, 32-k stage ch, part p,
-// lane l (row 16 j + l % 16, k 32 ch + 8 (l / 16) .. + 8), 16 bytes each.
-// Rows past N and k past Kp are zeros.
+// the wide kernel's lanes read them: 16-row tile j, 32-k stage ch, part p of
+// `parts`, lane l (row 16 j + l % 16, k 32 ch + 8 (l / 16) .. + 8), 16 bytes
+// each.  Rows past N and k past Kp are zeros.  One part: *rest becomes 1 if
+// any second part is not zero.
 __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ wnk,
                                                             const int* __restrict__ wexp,
                                                             u32x4* __restrict__ dst, int N, int Kp,
-                                                            int nch, long long pieces) {
+                                                            int nch, long long pieces, int parts,
+                                                            int* __restrict__ rest) {
   const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= pieces) return;
   const int lane = static_cast<int>(i & 63);
@@ -850,11 +865,14 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restr
   u32x4 p0, p1;
   vks::split8(make_float4(at(0), at(1), at(2), at(3)), make_float4(at(4), at(5), at(6), at(7)), &p0,
               &p1);
-  dst[jc * 128 + lane] = p0;
-  dst[jc * 128 + 64 + lane] = p1;
+  dst[jc * parts * 64 + lane] = p0;
+  if (parts == 2)
+    dst[jc * 128 + 64 + lane] = p1;
+  else if (((p1[0] | p1[1] | p1[2] | p1[3]) & 0x7fff7fffu) != 0)
+    *rest = 1;
 }
 
-int split_weights(vk_linear* lin) {
+int split_weights(vk_linear* lin, bool f16_values) {
   if (lin->in_features % 4 != 0) return VK_OK;  // never on the wide kernel
   const long long ntiles = (static_cast<long long>(lin->out_features) + 15) / 16;
   const long long nch = (static_cast<long long>(lin->in_features) + KC - 1) / KC;
@@ -862,17 +880,30 @@ int split_weights(vk_linear* lin) {
   const long long blocks = (pieces + 255) / 256;
   VK_UNSUPPORTED_IF(blocks > 0x7fffffffLL, "linear too large");
   const int n = static_cast<int>(lin->out_features), kp = static_cast<int>(lin->k_pitch);
-  // one allocation: the parts, then the exponents
-  const size_t bytes = static_cast<size_t>(pieces) * 32;
-  VK_HIP(hipMalloc(&lin->weight_split, bytes + static_cast<size_t>(n) * sizeof(int)));
-  lin->weight_exp = reinterpret_cast<int*>(static_cast<char*>(lin->weight_split) + bytes);
-  hipLaunchKernelGGL(weight_exponent_kernel, dim3((n + 3) / 4), dim3(256), 0, nullptr,
-                     lin->weight_nk, lin->weight_exp, n, kp);
-  VK_TRY(check_launch("weight_exponent_kernel"));
-  hipLaunchKernelGGL(split_weights_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                     nullptr, lin->weight_nk, lin->weight_exp,
-                     static_cast<u32x4*>(lin->weight_split), n, kp, static_cast<int>(nch), pieces);
-  VK_TRY(check_launch("split_weights_kernel"));
+  // f16 values have one part unless a column's range is wider than f16's
+  // (its smallest values then leave remainders): tried first, and split in two
+  // where the kernel finds a remainder.
+  for (int parts = f16_values ? 1 : 2; parts <= 2; ++parts) {
+    // one allocation: the parts, the exponents, the remainder flag
+    const size_t bytes = static_cast<size_t>(pieces) * 16 * parts;
+    VK_HIP(hipMalloc(&lin->weight_split, bytes + (static_cast<size_t>(n) + 1) * sizeof(int)));
+    lin->weight_exp = reinterpret_cast<int*>(static_cast<char*>(lin->weight_split) + bytes);
+    lin->weight_parts = parts;
+    hipLaunchKernelGGL(weight_exponent_kernel, dim3((n + 3) / 4), dim3(256), 0, nullptr,
+                       lin->weight_nk, lin->weight_exp, n, kp);
+    VK_TRY(check_launch("weight_exponent_kernel"));
+    hipLaunchKernelGGL(split_weights_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
+                       nullptr, lin->weight_nk, lin->weight_exp,
+                       static_cast<u32x4*>(lin->weight_split), n, kp, static_cast<int>(nch),
+                       pieces, parts, lin->weight_exp + n);
+    VK_TRY(check_launch("split_weights_kernel"));
+    if (parts == 2) break;
+    int rest = 0;
+    VK_HIP(hipMemcpy(&rest, lin->weight_exp + n, sizeof(int), hipMemcpyDeviceToHost));
+    if (!rest) return VK_OK;
+    VK_HIP(hipFree(lin->weight_split));
+    lin->weight_split = nullptr;
+  }
   VK_HIP(hipStreamSynchronize(nullptr));
   return VK_OK;
 }

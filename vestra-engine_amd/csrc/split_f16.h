@@ -17,6 +17,9 @@
 //    a NaN, and so is every sum that x enters (is_finite below);
 //  * a row (the values of one sum) that is small as a whole, so that the floor
 //    counts: its largest |x| is below kRowMin and not 0.
+// What stays: in a row of ordinary values, one below 2^-13 is held to 2^-36
+// (not to 2^-23 of itself), which a sum shows only where that value's weight is
+// thousands of times the others'.
 #pragma once
 
 #include "common.h"

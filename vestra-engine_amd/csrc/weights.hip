@@ -41,7 +41,7 @@ int make_linear(vk_runtime* rt, size_t in, size_t out, const std::vector<float>&
   lin->out_features = out;
   lin->k_pitch = (in + kKAlign - 1) / kKAlign * kKAlign;
   int s = alloc_copy(wnk.data(), lin->k_pitch * out, &lin->weight_nk);
-  if (s == VK_OK) s = vk::split_weights(lin);
+  if (s == VK_OK) s = vk::split_weights(lin, false);
   if (s == VK_OK) s = vk::prepare_patch_filter(rt, lin);
   if (s == VK_OK) s = alloc_copy(bias, out, &lin->bias);
   if (s == VK_OK && ls) s = alloc_copy(ls, out, &lin->ls_gamma);
@@ -150,7 +150,7 @@ int make_linear_stored(vk_runtime* rt, size_t in, size_t out, int src_kind, bool
     if (s == VK_OK && se != hipSuccess) s = vk::hip_fail(se, "hipStreamSynchronize");
     (void)hipFree(raw);
   }
-  if (s == VK_OK) s = vk::split_weights(lin);
+  if (s == VK_OK) s = vk::split_weights(lin, src_kind == kSrcF16);
   if (s == VK_OK) s = alloc_copy(bias, out, &lin->bias);
   if (s == VK_OK && ls) s = alloc_copy(ls, out, &lin->ls_gamma);
   if (s != VK_OK) {
