@@ -19,7 +19,8 @@ value = algorithmic bytes of every launched kernel / measured step time
 the oracle timed on the host cores as the CPU baseline, and -- beside the
 path -- the fused projection epilogues, the attention core and the whole
 device-resident block (projections and attention included) with their
-F32-MFMA rates.
+rates over the F32 matrix peak (a fraction above 1: they run F32 products on
+the f16 matrix cores).
 """
 import argparse
 import json
@@ -705,7 +706,7 @@ def vitl_timing(rt, rng, reps=3):
 
 
 def attention_timing(rt, rng, iters):
-    """The attention core (softmax(Q K^T / 8) V, F32 MFMA, online softmax) at
+    """The attention core (softmax(Q K^T / 8) V, F32 in and out, online softmax) at
     the path's shapes: one image (12 heads of 866 tokens), a local layer of
     the 12-view batch (144 sequences of 866 tokens), a global layer (12 heads
     over the flattened 10,392 rows) and the ViT-L 1008x672 image (16 heads

@@ -361,8 +361,8 @@ int vk_dequantize_q8_0_f32(vk_runtime* rt, const vk_tensor* blocks, size_t n,
                            vk_tensor* dst);
 int vk_linear_destroy(vk_linear* lin);
 size_t vk_linear_input_features(const vk_linear* lin);
-/* CudaLinearF32::run(x, rows): y = (x @ W + b) [* gamma], F32 MFMA with f32
- * accumulation.  New tensor [rows, out]. */
+/* CudaLinearF32::run(x, rows): y = (x @ W + b) [* gamma], f32 in and out
+ * with f32 accumulation.  New tensor [rows, out]. */
 int vk_linear_run_f32(vk_runtime* rt, const vk_linear* lin, const vk_tensor* x,
                       size_t rows, vk_tensor** out);
 /* The same into a caller tensor out [rows, out] (no allocation; capturable

@@ -708,10 +708,9 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __res
 
 // Key splits a caller must be ready to provide for: 1 where the shape never
 // splits (it can be captured before any eager call of its kind).  This is the
-// interface's rule, fixed apart from the splits that are taken: 64-query
-// tiles of fewer than two
-// workgroups per CU split to about two (at least two key blocks each, at most
-// 8); fuller grids where a model of 2.2 us per key block of the busiest CU,
+// interface's rule, fixed apart from the splits that are taken: 64-query tiles
+// of fewer than two workgroups per CU split to about two (at least two key
+// blocks each, at most 8); fuller grids where a model of 2.2 us per key block of the busiest CU,
 // the partial results' traffic at 5.5 TB/s and 3 us for the merge pass puts a
 // split at least 1% below the unsplit launch.
 int key_splits_to_provide(int cus, size_t sequences, size_t n) {

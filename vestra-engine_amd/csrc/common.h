@@ -266,13 +266,13 @@ enum LinearEpilogue {
 };
 }  // namespace linear_epilogue
 
-// The wide-tile linear (128 x 128, 64 x 128 or 64 x 64 tiles, split-K for
-// few rows) for K % 4 == 0 and a 16-byte aligned x (linear.hip);
-// the head-major layouts of LinearArgs need it.
 constexpr int kSplitK = 32;  // k of one stage of the wide kernel
 // Most floats of split-K partial sums: the allocation-free entry point's
 // scratch, so a plan that splits always fits it.
 constexpr long long kMaxPartialFloats = 8LL << 20;
+// The wide-tile linear (128 x 256 to 64 x 64 tiles, split-K for few rows) for
+// K % 4 == 0 and a 16-byte aligned x (linear.hip); the head-major layouts of
+// LinearArgs need it.
 // `partial` / `partial_floats`: the caller's buffer for split-K partial
 // sums (nothing is allocated; a plan that needs more is refused); null: the
 // runtime's work buffer, grown as needed.

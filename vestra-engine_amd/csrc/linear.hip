@@ -11,9 +11,8 @@
 //
 //  * A (activations, f32) is read by raw buffer loads one stage ahead, split
 //    by the thread that loaded it and staged through LDS as [row][part][32 k]
-//    f16 rows with a pitch of 144 bytes (16 x odd: the 16 rows of a fragment
-//    read start on 16 distinct 4-bank groups).  Two buffers: one barrier a
-//    stage.
+//    f16 rows with a pitch of 144 bytes (16 x odd).  Two buffers: one barrier
+//    a stage.
 //  * B (weights) was split when the linear was prepared, each column scaled
 //    by a power of two, into fragment order (split_weights): a wave's operand
 //    of one 16-column tile and part is 1 KiB that its 64 lanes read in order,
@@ -150,9 +149,9 @@ __device__ __forceinline__ float4 qk_head_row(const LinearArgs& g, float4 v, int
       v, l, gm, bt, py, px, g.qkn.table, g.qkn.table_max, g.qkn.eps);
 }
 
-// Most split-K slices a sum pass reads (choose_plan and
-// slices_to_provide).  The sum passes are instantiated for split-count buckets SPB
-// of 2, 4 and 8 (split_bucket).
+// Most split-K slices a sum pass reads (choose_plan and slices_to_provide).
+// The sum passes are instantiated for split-count buckets SPB of 2, 4 and 8
+// (split_bucket).
 constexpr int kMaxSplits = 8;
 constexpr int split_bucket(int splits) { return splits <= 2 ? 2 : (splits <= 4 ? 4 : 8); }
 
@@ -748,7 +747,6 @@ Plan choose_plan(long long cus, int M, int N, int K, int provided) {
                                {64, 64, 0.26, 0.0, kAlone}};
   const int nch = (K + KC - 1) / KC;
   const long long mn = static_cast<long long>(M) * N;
-  // the shortest run is kMaxStages or, if the slices do not allow that, 1 / max
   const auto may = [&](int sp) {
     return sp == 1 || (provided > 1 && sp <= kMaxSplits && 4 * sp <= nch &&
                        (sp <= provided || sp * mn <= kMaxPartialFloats));

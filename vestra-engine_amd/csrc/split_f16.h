@@ -9,7 +9,7 @@
 // the one left out is at most 2^-22 |x y| (rms about 2^-25).  The products are
 // exact, and main rounds once per 32 of k where the F32 matrix instruction
 // rounds once per 4: sums come out closer to the 64-bit values than from F32
-// products (K = 768: 1.4e-7 against 3.5-5.0e-7 relative), and
+// products (K = 768: 2.0e-7 against 3.5-5.0e-7 relative), and
 // v_mfma_f32_16x16x32_f16 runs 16 times the F32 rate for three products.
 //
 // What the split cannot hold is found and computed from the f32 values:
