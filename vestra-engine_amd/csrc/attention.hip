@@ -67,6 +67,8 @@ constexpr float kQScale = 0.125f * 1.44269504088896341f;  // log2(e) / sqrt(64)
 constexpr float kKvUp = 256.0f, kQUp = 1024.0f, kSDown = 1.0f / 262144.0f;
 constexpr float kPBits = 11.0f, kPDown = 1.0f / 2048.0f, kSlack = 4.0f;
 constexpr float kODown = kPDown / kKvUp;
+// The largest |v| from which a run of keys is held (its floor is 2^-33).
+constexpr float kRowMin = 1.0f / 512.0f;
 constexpr int kFlush = 8;       // blocks between additions to the running total
 constexpr int kRowBytes = 272;  // LDS pitch of 64 values: 2 parts x 128 bytes + 16
 constexpr int kBufBytes = 2 * KB * kRowBytes;  // a block of K and of V
@@ -460,8 +462,7 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
     *reinterpret_cast<uint2*>(d + 128) = make_uint2(p1[0], p1[1]);
   };
   auto store_v = [&](int buf, const float4 (&vr)[4]) {
-    vmax = vks::max_abs8(vmax, vr[0], vr[1]);
-    vmax = vks::max_abs8(vmax, vr[2], vr[3]);
+    vmax = fmaxf(vmax, fmaxf(vks::max_abs8(vr[0], vr[1]), vks::max_abs8(vr[2], vr[3])));
     char* d = v_dst + buf * kBufBytes;
     store_v4(d, vr[0].x, vr[1].x, vr[2].x, vr[3].x);
     store_v4(d + kRowBytes, vr[0].y, vr[1].y, vr[2].y, vr[3].y);
@@ -607,7 +608,7 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
 #pragma unroll
     for (int r = 0; r < 16; ++r) odd |= live && !vks::is_finite(total[dt][r]);
   // V is judged by the largest value of the run: two bits a wave
-  const bool big = vmax >= vks::kRowMin, some = vmax != 0.0f;
+  const bool big = vmax >= kRowMin, some = vmax != 0.0f;
   const int bits = (__builtin_amdgcn_ballot_w64(odd) ? 1 : 0) |
                    (__builtin_amdgcn_ballot_w64(big) ? 2 : 0) |
                    (__builtin_amdgcn_ballot_w64(some) ? 4 : 0);

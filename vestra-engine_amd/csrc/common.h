@@ -68,7 +68,10 @@ struct vk_linear {
   // The rows as f16 parts in the wide linear's fragment order, each row
   // scaled by 2^weight_exp (split_weights), for in_features % 4 == 0.
   void* weight_split = nullptr;
-  int* weight_exp = nullptr;   // [out], in weight_split's allocation
+  // In its allocation: the rows' exponents [out], and running counts of what
+  // the values are, [1 + stages][out].
+  int* weight_exp = nullptr;
+  uint2* weight_stat = nullptr;
   int weight_parts = 0;        // 1 where every second part is zero (f16 values)
   // For a 3x14x14 patch filter (in_features 588) only: the same rows with
   // the input dimension reordered (c, ky, kx) -> (ky, kx, c), the order in
@@ -222,7 +225,8 @@ struct LinearArgs {
   const float* x;     // [M, K]
   const float* wnk;   // [N, Kp], K contiguous, zero beyond K
   const void* wsplit; // its f16 parts (vk_linear::weight_split) and
-  const int* wexp;    // their rows' exponents, linear.hip only
+  const int* wexp;    // their rows' exponents and counts, linear.hip only
+  const uint2* wstat;
   int wparts;         // parts of a weight (vk_linear::weight_parts)
   const float* bias;  // [N]
   const float* ls;    // [N] or null

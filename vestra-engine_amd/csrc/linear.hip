@@ -48,10 +48,35 @@
 // (vkq::qk_row_transform) before storing the row head-major.  The values and
 // the code path are those of the separate pass, so the bits are too.
 //
-// A tile that the split cannot hold (a sum that is not finite, or a row whose
-// values are all tiny, split_f16.h) is computed again by the same workgroup
-// with F32 matrix instructions on the f32 operands.  A split-K workgroup
-// decides for its own run of k.
+// Every output is either the split's sum or, where the split may hold its
+// terms less well than F32 does, an F32 one: the wave computes the 16 rows of
+// its columns again with F32 matrix instructions on the f32 operands and takes
+// the outputs in question from there.  Which they are depends on the output's
+// own row and column alone (and the split-K run), so no other row or column of
+// a tile changes its bits:
+//  * the sum is not finite;
+//  * the floor of 2^-36 could show.  Rows of A are scaled by a power of two that
+//    brings their typical value (of two stages) into [2^6, 2^7), columns of B to
+//    [2^10, 2^11).  In groups of 8 k, with G groups in the run, a row counts the
+//    groups found to reach 1 (big; three of the eight values are looked at) and
+//    those with a value below 2^-13 (tiny), a column its groups of weights all of
+//    at least 8 (dense) and its weights below 2^-13 that their parts do not hold
+//    exactly (tiny).  Then
+//      the floor's share of a sum   <= 2^-24 (4 tiny_row + 16 tiny_col),
+//      the sum of its |terms|  s    >= 8 (big + dense - G)  and  >= |sum|,
+//    the first bound because at least big + dense - G groups hold a value of at
+//    least 1 whose weight is at least 8.  Taken again unless one of the two
+//    reaches 4 tiny_row + 16 tiny_col: the floor then stays below 2^-24 s;
+//  * a sum of few terms, which F32 adds with next to no rounding (a one-hot
+//    column copies): fewer than 8 groups of the row reach 1, or of the column 8.
+// Ordinary rows (layer-normalised, GELU outputs, attention outputs) and dense
+// columns pass as a whole; then an output costs only the test that it is finite.
+// The scale and the counts take 0.5 to 0.9 us of a launch of one image (866 x 768
+// -> 2304 18.2 -> 19.2 us) and 1 to 3% of the large ones.  Rows of any scale up to
+// f32's run at that speed (x 1e-6: 20.6 us; judged by a fixed scale and taken
+// again tile by tile 69).  A launch that takes every output again (NaN
+// throughout; eight decades of sizes in every row) costs about 1.8 times one on
+// F32 matrix instructions alone: 10,392 x 768 -> 3072 740 us against 386.
 //
 // Tiles are numbered XCD-major in groups of at most 1,024 rows (tile_of): the
 // workgroups an XCD holds at one time then share both a slice of A and one
@@ -70,6 +95,17 @@ using vks::u32x4;
 constexpr int KC = vk::kSplitK;    // k of one stage (and of one MFMA)
 // Waves of a tile: one per 32 columns, at least four.
 constexpr int waves_for(int tn) { return tn == 256 ? 8 : 4; }
+// Values below kTiny have the split's floor; groups of 8 k with a value of A of
+// at least kXBig, or weights of at least kWBig, count as big or dense.
+constexpr float kTiny = 1.0f / 8192.0f, kXBig = 1.0f, kWBig = 8.0f;
+// A row's typical value is brought to [2^kRowBits, 2 x that), its largest one
+// (of those looked at) below 2^(kRowMaxBits + 1).
+constexpr int kRowBits = 6, kRowMaxBits = 13;
+constexpr int kFewGroups = 8;      // sums of fewer groups than this are F32 sums
+// The linears of the split: at least kFewGroups groups, counts of 16 bits.
+constexpr int kMinSplitK = 8 * kFewGroups, kMaxSplitK = 1 << 18;
+constexpr int kZeroColumn = 1 << 20;  // exponent of a column of zeros
+constexpr int kZeroRow = 0xffff;      // count of a row of zeros
 constexpr int kRowBytes = 144;     // LDS pitch of a row of A: 2 parts x 64 bytes + 16
 constexpr int kXsPitch = 68;       // f32 pitch of the Q/K epilogue's rows
 static_assert(kRowBytes % 16 == 0 && (kRowBytes / 16) % 2 == 1 && kRowBytes >= 4 * KC, "pitch");
@@ -197,11 +233,43 @@ __device__ __forceinline__ void tile_of(int t, int gmt, int gnt, int splits, int
   *split = rest / gnt;
 }
 
+// Largest value and sum over the four lanes 4 i .. 4 i + 3 (a row's pieces).
+__device__ __forceinline__ uint32_t quad_other(uint32_t v, int step) {
+  const int x = static_cast<int>(v);  // quad_perm [1, 0, 3, 2] and [2, 3, 0, 1]
+  return static_cast<uint32_t>(step == 1 ? __builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, true)
+                                         : __builtin_amdgcn_mov_dpp(x, 0x4e, 0xf, 0xf, true));
+}
+
+__device__ __forceinline__ uint32_t quad_sum(uint32_t v) {
+  v += quad_other(v, 1);
+  return v + quad_other(v, 2);
+}
+
+__device__ __forceinline__ float quad_max(float v) {
+  v = fmaxf(v, __uint_as_float(quad_other(__float_as_uint(v), 1)));
+  return fmaxf(v, __uint_as_float(quad_other(__float_as_uint(v), 2)));
+}
+
 // NP: f16 parts of a weight.  Weights that are f16 values have one (the other
 // is all zeros, so the sums are the same): two products, half of B's bytes.
 //
 // KS: stages of 32 k per barrier (2 for the 64-row tiles, whose 12 or 24
 // MFMAs a wave and stage are too few to cover a load's latency).
+// What a column's weights are in stages [c_begin, c_end): groups of 8 k all of
+// at least kWBig, groups that reach it, weights with a floor (split_weights).
+struct ColumnRun {
+  int dense, any, tiny;
+};
+
+__device__ __forceinline__ ColumnRun column_run(const LinearArgs& g, int col, int c_begin,
+                                                int c_end) {
+  const uint2 a = g.wstat[static_cast<size_t>(c_begin) * g.N + col];
+  const uint2 b = g.wstat[static_cast<size_t>(c_end) * g.N + col];
+  return ColumnRun{static_cast<int>((b.x - a.x) & 0xffffu),
+                   static_cast<int>((b.x >> 16) - (a.x >> 16)) & 0xffff,
+                   static_cast<int>(b.y - a.y)};
+}
+
 template <int EPI, int LAY, int QKN, int TM, int TN, int KS, int NP>
 __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(LinearArgs g) {
   constexpr int kWaves = waves_for(TN), kThreads = 64 * kWaves;
@@ -219,6 +287,12 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   constexpr int kSmem = 2 * kBufBytes > kXsBytes ? 2 * kBufBytes : kXsBytes;
   __shared__ __align__(16) char smem[kSmem];
 
+  // The arguments lie in host memory: a first read of one of their cache lines
+  // takes about 2 us, so all lines are read at once here and not one after the
+  // other where the code below first needs them.
+  asm volatile("" ::"s"(g.x), "s"(g.M), "s"(g.qkn_mode), "s"(g.qkn.eps), "s"(g.ln_out),
+               "s"(gridDim.x));
+
   const int tid = threadIdx.x;
   __builtin_assume(tid < kThreads);
   const int wave = tid >> 6, lane = tid & 63;
@@ -228,8 +302,9 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   tile_of<TM>(vkd::xcd_tile(blockIdx.x, gridDim.x), gmt, gnt, g.splits, &mt, &nt, &split);
   const int m0 = mt * TM, n0 = nt * TN;
   const int nch = (g.K + KC - 1) / KC;
-  const int c_begin = static_cast<int>(static_cast<long long>(split) * nch / g.splits);
-  const int c_end = static_cast<int>(static_cast<long long>(split + 1) * nch / g.splits);
+  // split <= 8 and nch < 2^26: 32 bits hold the products
+  const int c_begin = static_cast<int>(static_cast<uint32_t>(split) * nch / g.splits);
+  const int c_end = static_cast<int>(static_cast<uint32_t>(split + 1) * nch / g.splits);
 
   // A: slot i of a thread is piece s = tid + 256 i: stage s / (4 TM), row
   // (s / 4) % TM, k 8 (s % 4) .. + 8 of that stage.  Rows past M read a
@@ -255,7 +330,7 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   float4 ra[kVA][2];
   // k past K, and stages past the split's end, read past the buffer, which
   // gives zeros.
-  auto load_a = [&](int ch0) {
+  auto load_a = [&](int ch0, float4 (&ra)[kVA][2]) {
 #pragma unroll
     for (int i = 0; i < kVA; ++i) {
       const int at = ch0 + slot_stage(i);
@@ -268,15 +343,21 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
             a_rsrc, 8 * piece + 4 * h < left ? a_off[i] + 16u * h : 0xfffffff0u, base);
     }
   };
-  float amax[kVA];  // largest |x| of the slot's pieces so far
-#pragma unroll
-  for (int i = 0; i < kVA; ++i) amax[i] = 0.0f;
+  // Per row of the thread's slots: its scale, the groups counted, the bits of any
+  // first part.
+  constexpr int kVR = kVA / KS;
+  float rscale[kVR];
+  uint32_t rbig[kVR], rtiny[kVR], rany[kVR];
   auto store_a = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < kVA; ++i) {
-      amax[i] = vks::max_abs8(amax[i], ra[i][0], ra[i][1]);
+      const int rr = i % kVR;
+      const float4 x = vks::scale4(ra[i][0], rscale[rr]), y = vks::scale4(ra[i][1], rscale[rr]);
+      rbig[rr] += fmaxf(fmaxf(fabsf(x.x), fabsf(x.w)), fabsf(y.z)) >= kXBig;  // three of eight
+      rtiny[rr] += vks::min_abs8(x, y) < kTiny;
       u32x4 p0, p1;
-      vks::split8(ra[i][0], ra[i][1], &p0, &p1);
+      vks::split8(x, y, &p0, &p1);
+      rany[rr] |= p0[0] | p0[1] | p0[2] | p0[3];
       char* d = smem + buf * kBufBytes + slot_stage(i) * kStageBytes + slot_row(i) * kRowBytes +
                 16 * piece;
       *reinterpret_cast<u32x4*>(d) = p0;
@@ -342,27 +423,65 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
     }
   };
 
-  // One stage: split and store what was loaded a stage earlier, issue the
-  // next stage's loads, run this one's MFMAs.  A buffer is written again two
-  // stages after it was read, with a barrier in between.
+  // One stage: run its MFMAs, split and store the next one and issue the loads
+  // of the one after.  A buffer is written again in the stage after the one
+  // that read it, with a barrier in between.
   u32x4 b0[KS][NU][NP], b1[KS][NU][NP];
-  load_a(c_begin);
-  load_b(c_begin, b0);
-  int ch = c_begin;
-  for (; ch + KS < c_end; ch += 2 * KS) {
+  const bool split_k = g.K >= kMinSplitK && g.K < kMaxSplitK;  // else F32 throughout
+  const int groups = 4 * (c_end - c_begin);
+  auto col_of = [&](int u) { return n0 + wave * WN + u * 16 + (lane & 15); };
+  int cexp[NU];
+  ColumnRun cr[NU];
+  int ch = split_k ? c_begin : c_end;
+  if (split_k) {
+    load_a(c_begin, ra);
+    float4 rm[kVA][2];  // the run's middle, for the scale
+    load_a((c_begin + c_end) >> 1, rm);
+    load_b(c_begin, b0);
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int col = col_of(u) < g.N ? col_of(u) : g.N - 1;
+      cexp[u] = g.wexp[col];
+      cr[u] = column_run(g, col, c_begin, c_end);
+    }
+#pragma unroll
+    for (int i = 0; i < kVR; ++i) {
+      float m = 0.0f, t = 0.0f;
+#pragma unroll
+      for (int j = i; j < kVA; j += kVR) {
+        const float first = vks::max_abs8(ra[j][0], ra[j][1]);
+        const float mid = vks::max_abs8(rm[j][0], rm[j][1]);
+        m = fmaxf(m, fmaxf(first, mid));
+        t = fmaxf(t, fminf(first, mid));
+      }
+      m = quad_max(m);  // the four pieces of a row are adjacent lanes
+      t = quad_max(t);
+      // values in [2^(b - 127), 2^(b - 126)).  No value seen: the largest scale, by
+      // which every other f32 has a first part that is not 0.
+      const int bm = static_cast<int>(__float_as_uint(m) >> 23);
+      const int bt = t > 0.0f ? static_cast<int>(__float_as_uint(t) >> 23) : bm;
+      int e = kRowBits + 127 - bt;
+      e = e < kRowMaxBits + 127 - bm ? e : kRowMaxBits + 127 - bm;
+      e = bm == 255 ? 0 : (m == 0.0f || e > 126 ? 126 : e);
+      rscale[i] = __uint_as_float(static_cast<uint32_t>(127 + e) << 23);
+      rbig[i] = rtiny[i] = rany[i] = 0;
+    }
     store_a(0);
+    load_a(ch + KS, ra);
+  }
+  for (; ch + KS < c_end; ch += 2 * KS) {
     __syncthreads();
-    load_a(ch + KS);
     load_b(ch + KS, b1);
     mma(0, b0);
     store_a(1);
+    load_a(ch + 2 * KS, ra);
     __syncthreads();
-    load_a(ch + 2 * KS);
     load_b(ch + 2 * KS, b0);
     mma(1, b1);
+    if (ch + 2 * KS < c_end) store_a(0);
+    load_a(ch + 3 * KS, ra);
   }
   if (ch < c_end) {
-    store_a(0);
     __syncthreads();
     mma(0, b0);
   }
@@ -370,83 +489,156 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   // lane holds D[4 (lane / 16) + r][lane % 16] of each 16 x 16 tile
   const int g4 = lane >> 4, c16 = lane & 15;
   auto row_of = [&](int t, int r) { return m0 + t * 16 + 4 * g4 + r; };
-  auto col_of = [&](int u) { return n0 + wave * WN + u * 16 + c16; };
 
-  // The sums, and whether the split held everything that went into them.
-  bool odd = false;
+  // The sums.  Rows' counts and exponents meet in LDS.
+  int* row_exp = reinterpret_cast<int*>(smem);
+  int* row_cnt = row_exp + TM;
+  int* flags = row_cnt + TM;  // one per wave: a row that is not plain
+  bool look = !split_k;
+  if (split_k) {
 #pragma unroll
-  for (int u = 0; u < NU; ++u) {
-    const int e = -g.wexp[col_of(u) < g.N ? col_of(u) : g.N - 1];
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = __builtin_fmaf(corr[t][u][r], vks::kDown, acc[t][u][r]);
-        odd |= !vks::is_finite(v);
-        acc[t][u][r] = __builtin_amdgcn_ldexpf(v, e);
-      }
-  }
-#pragma unroll
-  for (int i = 0; i < kVA / KS; ++i) {  // the four pieces of a row are adjacent lanes
-    float m = amax[i];
-#pragma unroll
-    for (int s = 1; s < KS; ++s) m = fmaxf(m, amax[i + s * (kVA / KS)]);
-    m = fmaxf(m, __shfl_xor(m, 1, 64));
-    m = fmaxf(m, __shfl_xor(m, 2, 64));
-    odd |= m < vks::kRowMin && m != 0.0f;
-  }
-  int* flags = reinterpret_cast<int*>(smem);  // one per wave
-  __syncthreads();  // every wave is done with the last stage
-  const bool wave_odd = __builtin_amdgcn_ballot_w64(odd) != 0;
-  if (lane == 0) flags[wave] = wave_odd;
-  __syncthreads();
-  int any = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) any |= flags[w];
-  if (__builtin_expect(any, 0)) {
-    // The tile again, with F32 matrix instructions (fragment order: lane
-    // group g4 holds k = 16 b + 4 g4 + j of block b in component j).
-    constexpr int kPitchF = kRowBytes / 4;
-    float* As = reinterpret_cast<float*>(smem);
+    for (int u = 0; u < NU; ++u)
+      look |= (cexp[u] != kZeroColumn) &
+              ((cr[u].any < kFewGroups) |
+               (8 * (cr[u].dense - groups) - 16 * cr[u].tiny < -6 * groups));
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int u = 0; u < NU; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int ch = c_begin; ch < c_end; ++ch) {
-      __syncthreads();
-#pragma unroll 1
-      for (int s = tid; s < TM * 8; s += kThreads) {
-        const int row = s >> 3, k = ch * KC + 4 * (s & 7);
-        const int gm = m0 + row < g.M ? m0 + row : g.M - 1;
-        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-        const size_t at = LAY == kAHnd ? (static_cast<size_t>(k >> 6) * g.M + gm) * 64 + (k & 63)
-                                       : static_cast<size_t>(gm) * g.K + k;
-        *reinterpret_cast<float4*>(As + row * kPitchF + 4 * (s & 7)) =
-            k < g.K ? *reinterpret_cast<const float4*>(g.x + at) : z;
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          acc[t][u][r] = __builtin_fmaf(corr[t][u][r], vks::kDown, acc[t][u][r]);
+          look |= !vks::is_finite(acc[t][u][r]);
+        }
+    __syncthreads();  // every wave is done with the last stage
+    bool plain_rows = true;
+#pragma unroll
+    for (int i = 0; i < kVR; ++i) {
+      // a stage past the run's end counted one piece of zeros
+      const int tiny = static_cast<int>(
+          quad_sum(rtiny[i] - ((c_end - c_begin) % KS != 0 ? 1u : 0u)));
+      const int big = static_cast<int>(quad_sum(rbig[i]));
+      const uint32_t any = quad_sum(rany[i] & 0x7fff7fffu ? 1u : 0u);
+      plain_rows &= any == 0 || (big >= kFewGroups && 8 * big - 4 * tiny >= 6 * groups);
+      if (piece == 0) {
+        row_exp[slot_row(i)] = static_cast<int>(__float_as_uint(rscale[i]) >> 23) - 127;
+        row_cnt[slot_row(i)] = any == 0 ? kZeroRow : tiny << 16 | big;
       }
-      __syncthreads();
-#pragma unroll 1
-      for (int b = 0; b < 2; ++b) {
-        const int k = ch * KC + 16 * b + 4 * g4;
-        f32x4 w[NU];
+    }
+    const bool rows_look = __builtin_amdgcn_ballot_w64(!plain_rows) != 0;
+    if (lane == 0) flags[wave] = rows_look;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) look |= flags[w] != 0;
+  }
+  // exponents of rows 16 t + 4 g4 .. + 4
+  auto row4 = [&](const int* p, int t) {
+    return *reinterpret_cast<const int4*>(p + t * 16 + 4 * g4);
+  };
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(look) == 0, 1)) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const int4 e4 = row4(row_exp, t);
+      const int e[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          acc[t][u][r] = __builtin_amdgcn_ldexpf(acc[t][u][r], -e[r] - cexp[u]);
+    }
+  } else {
+    // Output by output; 64 rows with any to take again are computed in F32
+    // (fragment order: lane group g4 holds k = 16 b + 4 g4 + j of block b in
+    // component j), straight from memory and without a barrier.
+    const float* wrow[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int col = col_of(u) < g.N ? col_of(u) : g.N - 1;
+      wrow[u] = g.wnk + static_cast<size_t>(col) * g.Kp;
+    }
+#pragma unroll
+    for (int t0 = 0; t0 < MT; t0 += 4) {
+      uint32_t again[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        again[i] = 0xffffffffu;
+        if (!split_k) continue;
+        const int t = t0 + i;
+        const int4 e4 = row4(row_exp, t), c4 = row4(row_cnt, t);
+        const int e[4] = {e4.x, e4.y, e4.z, e4.w}, c[4] = {c4.x, c4.y, c4.z, c4.w};
+        again[i] = 0;
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float v = acc[t][u][r];
+            const int big = c[r] & 0xffff, tiny = (c[r] >> 16) & 0xffff;
+            const int need = 4 * tiny + 16 * cr[u].tiny;
+            const bool held =
+                c[r] == kZeroRow || cexp[u] == kZeroColumn ||
+                (big >= kFewGroups && cr[u].any >= kFewGroups &&
+                 (8 * (big + cr[u].dense - groups) >= need || fabsf(v) >= static_cast<float>(need)));
+            if (!held || !vks::is_finite(v)) again[i] |= 1u << (4 * u + r);
+            acc[t][u][r] = __builtin_amdgcn_ldexpf(v, -e[r] - cexp[u]);
+          }
+      }
+      if (__builtin_amdgcn_ballot_w64((again[0] | again[1] | again[2] | again[3]) != 0) == 0)
+        continue;
+      const float* arow[4];  // the fragments' rows
+      f32x4 f[4][NU];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = m0 + (t0 + i) * 16 + c16;
+        arow[i] = g.x + static_cast<size_t>(row < g.M ? row : g.M - 1) * (LAY == kAHnd ? 64 : g.K);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) f[i][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      // 16 k ahead in registers; k past K multiplies zeros
+      f32x4 a[4], w[NU];
+      auto fetch = [&](int b) {
+        const int k = 16 * b + 4 * g4;
+        const int ck = k < g.K ? k : 0;
+        const size_t at = LAY == kAHnd ? static_cast<size_t>(ck >> 6) * g.M * 64 + (ck & 63)
+                                       : static_cast<size_t>(ck);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = *reinterpret_cast<const f32x4*>(arow[i] + at);
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-          const int col = col_of(u) < g.N ? col_of(u) : g.N - 1;
-          w[u] = k < g.Kp ? *reinterpret_cast<const f32x4*>(g.wnk + static_cast<size_t>(col) * g.Kp + k)
-                          : f32x4{0.f, 0.f, 0.f, 0.f};
+          w[u] = *reinterpret_cast<const f32x4*>(wrow[u] + ck);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[u][j] = k < g.K ? w[u][j] : 0.0f;
         }
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          const f32x4 a =
-              *reinterpret_cast<const f32x4*>(As + (t * 16 + c16) * kPitchF + 16 * b + 4 * g4);
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int j = 0; j < 4; ++j) a[i][j] = k < g.K ? a[i][j] : 0.0f;
+      };
+      const int b_end = 2 * c_end < (g.K + 15) / 16 ? 2 * c_end : (g.K + 15) / 16;
+      fetch(2 * c_begin);
+#pragma unroll 1
+      for (int b = 2 * c_begin; b < b_end; ++b) {
+        f32x4 ca[4], cw[NU];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ca[i] = a[i];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) cw[u] = w[u];
+        fetch(b + 1 < b_end ? b + 1 : b);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int u = 0; u < NU; ++u)
-              acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], w[u][j], acc[t][u], 0, 0, 0);
-        }
+              f[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(ca[i][j], cw[u][j], f[i][u], 0, 0, 0);
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if ((again[i] >> (4 * u + r)) & 1) acc[t0 + i][u][r] = f[i][u][r];
     }
   }
 
@@ -817,7 +1009,7 @@ void launch_pair(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 gri
 
 // Exponent of each weight column for the split: wexp[n] = e brings the
 // column's largest |w| to 2^e |w| in [2^10, 2^11), so that every value down to
-// 2^-24 of it has both parts (0 for a column of zeros).
+// 2^-24 of it has both parts (kZeroColumn for a column of zeros).
 __global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __restrict__ wnk,
                                                               int* __restrict__ wexp, int N,
                                                               int Kp) {
@@ -836,19 +1028,22 @@ __global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __res
   }
   int e = 0;
   if (m) (void)frexpf(__uint_as_float(m), &e);  // m in [2^(e-1), 2^e)
-  if (lane == 0) wexp[row] = m ? 11 - e : 0;
+  if (lane == 0) wexp[row] = m ? 11 - e : kZeroColumn;
 }
 
 // The f16 parts of the scaled rows 2^wexp[n] wnk[n] of [N, Kp] in the order
 // the wide kernel's lanes read them: 16-row tile j, 32-k stage ch, part p of
 // `parts`, lane l (row 16 j + l % 16, k 32 ch + 8 (l / 16) .. + 8), 16 bytes
 // each.  Rows past N and k past Kp are zeros.  One part: *rest becomes 1 if
-// any second part is not zero.
+// any second part is not zero.  stat[1 + ch][n] counts the stage's groups of 8 k
+// of row n: x the dense ones and, in the high half, those that reach kWBig; y
+// the weights below kTiny that the parts do not hold (column_run).
 __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ wnk,
                                                             const int* __restrict__ wexp,
                                                             u32x4* __restrict__ dst, int N, int Kp,
                                                             int nch, long long pieces, int parts,
-                                                            int* __restrict__ rest) {
+                                                            int* __restrict__ rest,
+                                                            uint2* __restrict__ stat) {
   const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= pieces) return;
   const int lane = static_cast<int>(i & 63);
@@ -860,14 +1055,50 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restr
   auto at = [&](int h) {
     return row < N && k0 + h < Kp ? ldexpf(wnk[static_cast<size_t>(row) * Kp + k0 + h], e) : 0.0f;
   };
+  const float4 x = make_float4(at(0), at(1), at(2), at(3));
+  const float4 y = make_float4(at(4), at(5), at(6), at(7));
   u32x4 p0, p1;
-  vks::split8(make_float4(at(0), at(1), at(2), at(3)), make_float4(at(4), at(5), at(6), at(7)), &p0,
-              &p1);
+  vks::split8(x, y, &p0, &p1);
+  const float w8[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+  uint32_t tiny = 0;
+#pragma unroll
+  for (int h = 0; h < 8; ++h) {
+    const auto part = [&](const u32x4& p) {
+      return static_cast<float>(__builtin_bit_cast(vks::f16x8, p)[h]);
+    };
+    tiny += fabsf(w8[h]) < kTiny && __builtin_fmaf(part(p1), vks::kDown, part(p0)) != w8[h];
+  }
+  uint32_t groups = (vks::min_abs8(x, y) >= kWBig ? 1u : 0u) +
+                    (vks::max_abs8(x, y) >= kWBig ? 0x10000u : 0u);
+#pragma unroll
+  for (int s = 16; s < 64; s <<= 1) {  // the stage's four groups of a row
+    groups += static_cast<uint32_t>(__shfl_xor(static_cast<int>(groups), s, 64));
+    tiny += static_cast<uint32_t>(__shfl_xor(static_cast<int>(tiny), s, 64));
+  }
+  if (lane < 16 && row < N) stat[static_cast<size_t>(ch + 1) * N + row] = make_uint2(groups, tiny);
   dst[jc * parts * 64 + lane] = p0;
   if (parts == 2)
     dst[jc * 128 + 64 + lane] = p1;
   else if (((p1[0] | p1[1] | p1[2] | p1[3]) & 0x7fff7fffu) != 0)
     *rest = 1;
+}
+
+// Running totals of the stages' counts: stat[ch] becomes those of the stages
+// before ch.
+__global__ __launch_bounds__(256) void stage_totals_kernel(uint2* __restrict__ stat, int N,
+                                                           int nch) {
+  const int n = blockIdx.x * 256 + threadIdx.x;
+  if (n >= N) return;
+  uint2 sum = make_uint2(0, 0);
+  stat[n] = sum;
+  for (int ch = 1; ch <= nch; ++ch) {
+    uint2* p = stat + static_cast<size_t>(ch) * N + n;
+    const uint2 v = *p;
+    // the halves of x wrap on their own (read back as differences)
+    sum = make_uint2(((sum.x + v.x) & 0xffffu) | ((sum.x & 0xffff0000u) + (v.x & 0xffff0000u)),
+                     sum.y + v.y);
+    *p = sum;
+  }
 }
 
 int split_weights(vk_linear* lin, bool f16_values) {
@@ -882,10 +1113,14 @@ int split_weights(vk_linear* lin, bool f16_values) {
   // (its smallest values then leave remainders): tried first, and split in two
   // where the kernel finds a remainder.
   for (int parts = f16_values ? 1 : 2; parts <= 2; ++parts) {
-    // one allocation: the parts, the exponents, the remainder flag
+    // one allocation: the parts, the stages' counts, the exponents, the remainder flag
     const size_t bytes = static_cast<size_t>(pieces) * 16 * parts;
-    VK_HIP(hipMalloc(&lin->weight_split, bytes + (static_cast<size_t>(n) + 1) * sizeof(int)));
-    lin->weight_exp = reinterpret_cast<int*>(static_cast<char*>(lin->weight_split) + bytes);
+    const size_t stat_bytes = (static_cast<size_t>(nch) + 1) * n * sizeof(uint2);
+    VK_HIP(hipMalloc(&lin->weight_split,
+                     bytes + stat_bytes + (static_cast<size_t>(n) + 1) * sizeof(int)));
+    char* base = static_cast<char*>(lin->weight_split);
+    lin->weight_stat = reinterpret_cast<uint2*>(base + bytes);
+    lin->weight_exp = reinterpret_cast<int*>(base + bytes + stat_bytes);
     lin->weight_parts = parts;
     hipLaunchKernelGGL(weight_exponent_kernel, dim3((n + 3) / 4), dim3(256), 0, nullptr,
                        lin->weight_nk, lin->weight_exp, n, kp);
@@ -893,8 +1128,11 @@ int split_weights(vk_linear* lin, bool f16_values) {
     hipLaunchKernelGGL(split_weights_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
                        nullptr, lin->weight_nk, lin->weight_exp,
                        static_cast<u32x4*>(lin->weight_split), n, kp, static_cast<int>(nch),
-                       pieces, parts, lin->weight_exp + n);
+                       pieces, parts, lin->weight_exp + n, lin->weight_stat);
     VK_TRY(check_launch("split_weights_kernel"));
+    hipLaunchKernelGGL(stage_totals_kernel, dim3((n + 255) / 256), dim3(256), 0, nullptr,
+                       lin->weight_stat, n, static_cast<int>(nch));
+    VK_TRY(check_launch("stage_totals_kernel"));
     if (parts == 2) break;
     int rest = 0;
     VK_HIP(hipMemcpy(&rest, lin->weight_exp + n, sizeof(int), hipMemcpyDeviceToHost));
@@ -909,9 +1147,9 @@ int split_weights(vk_linear* lin, bool f16_values) {
 int launch_linear_wide(vk_runtime* rt, const LinearArgs& g0, int epi, float* partial,
                        size_t partial_floats) {
   LinearArgs g = g0;
-  // An output element's bits depend on the plan (its split count) and the
-  // plan on (M, N, K) alone, so every layout and epilogue of one shape gives
-  // the same bits.
+  // An output element's bits depend on its row of x, its column of W and the
+  // plan, and the plan on (M, N, K) alone, so every layout and epilogue of one
+  // shape gives the same bits.
   const long long cus = rt->cu_count > 0 ? rt->cu_count : 256;
   const int provided = slices_to_provide(cus, g.M, g.N, g.K);
   const Plan plan = choose_plan(cus, g.M, g.N, g.K, provided);

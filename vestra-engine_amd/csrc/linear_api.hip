@@ -175,6 +175,7 @@ LinearArgs linear_args(const vk_linear* lin, const vk_tensor* x, size_t rows, vk
   g.wnk = lin->weight_nk;
   g.wsplit = lin->weight_split;
   g.wexp = lin->weight_exp;
+  g.wstat = lin->weight_stat;
   g.wparts = lin->weight_parts;
   g.bias = lin->bias;
   g.ls = lin->ls_gamma;
@@ -210,6 +211,7 @@ int launch_linear(vk_runtime* rt, const vk_linear* lin, const vk_tensor* x, size
   g.wnk = lin->weight_nk;
   g.wsplit = lin->weight_split;
   g.wexp = lin->weight_exp;
+  g.wstat = lin->weight_stat;
   g.wparts = lin->weight_parts;
   g.bias = lin->bias;
   g.ls = lin->ls_gamma;

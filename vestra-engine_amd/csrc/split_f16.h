@@ -12,14 +12,13 @@
 // products (K = 768: 2.0e-7 against 3.5-5.0e-7 relative), and
 // v_mfma_f32_16x16x32_f16 runs 16 times the F32 rate for three products.
 //
-// What the split cannot hold is found and computed from the f32 values:
-//  * |x| beyond f16's largest value, infinities and NaN: x0 is an infinity or
-//    a NaN, and so is every sum that x enters (is_finite below);
-//  * a row (the values of one sum) that is small as a whole, so that the floor
-//    counts: its largest |x| is below kRowMin and not 0.
-// What stays: in a row of ordinary values, one below 2^-13 is held to 2^-36
-// (not to 2^-23 of itself), which a sum shows only where that value's weight is
-// thousands of times the others'.
+// What the split holds less well than F32, and who answers for it:
+//  * values beyond f16's largest, infinities and NaN: x0 is an infinity or a
+//    NaN, and so is every sum that x enters (is_finite below);
+//  * values below 2^-13: held to 2^-36, not to 2^-23 of themselves.  The
+//    linear counts them and proves, output by output, that the floor is below
+//    one F32 rounding of the sum's terms (linear.hip); the attention scales
+//    the columns of V and looks at every query's result (attention.hip).
 #pragma once
 
 #include "common.h"
@@ -35,10 +34,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kUp = 2048.0f;          // 2^11
 constexpr float kDown = 1.0f / 2048.0f;
-// Rows whose largest value is at least this hold the 2^-36 floor below
-// sqrt(K) 2^-27 of that value.
-constexpr float kRowMin = 1.0f / 512.0f;
-
 // Both parts of two values, packed (a in the low half).
 __device__ __forceinline__ void split2(float a, float b, uint32_t* p0, uint32_t* p1) {
   const f16x2 h = __builtin_convertvector((f32x2{a, b}), f16x2);
@@ -69,12 +64,23 @@ __device__ __forceinline__ void split2_plain(float a, float b, uint32_t* p0, uin
   *p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2));
 }
 
-// The largest |x| of eight values and m (NaN left out).
-__device__ __forceinline__ float max_abs8(float m, const float4& x, const float4& y) {
-  m = fmaxf(fmaxf(m, fabsf(x.x)), fabsf(x.y));
-  m = fmaxf(fmaxf(m, fabsf(x.z)), fabsf(x.w));
-  m = fmaxf(fmaxf(m, fabsf(y.x)), fabsf(y.y));
-  return fmaxf(fmaxf(m, fabsf(y.z)), fabsf(y.w));
+// The largest and the smallest |x| of eight values (NaN left out).
+__device__ __forceinline__ float max_abs8(const float4& x, const float4& y) {
+  float m = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fabsf(x.z));
+  m = fmaxf(fmaxf(m, fabsf(x.w)), fabsf(y.x));
+  m = fmaxf(fmaxf(m, fabsf(y.y)), fabsf(y.z));
+  return fmaxf(m, fabsf(y.w));
+}
+
+__device__ __forceinline__ float min_abs8(const float4& x, const float4& y) {
+  float m = fminf(fminf(fabsf(x.x), fabsf(x.y)), fabsf(x.z));
+  m = fminf(fminf(m, fabsf(x.w)), fabsf(y.x));
+  m = fminf(fminf(m, fabsf(y.y)), fabsf(y.z));
+  return fminf(m, fabsf(y.w));
+}
+
+__device__ __forceinline__ float4 scale4(const float4& x, float s) {
+  return make_float4(x.x * s, x.y * s, x.z * s, x.w * s);
 }
 
 __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
