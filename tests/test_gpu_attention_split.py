@@ -68,3 +68,17 @@ def test_infinities_and_nan_stay_in_their_sequence(rt, rng, s, n):
                       "columns beside a NaN")
     if s > 2:
         assert np.array_equal(got[2:], good[2:])
+
+
+# four waves unsplit, eight waves unsplit, four waves in three key splits, eight in three
+@pytest.mark.parametrize("s,n", [(250, 300), (40, 800), (12, 866), (12, 1732)])
+def test_a_neighbours_growing_maximum_changes_no_bits(rt, rng, s, n):
+    """A query's running maximum moves by its own scores alone."""
+    q, k, v = (normals(rng, s, n, 64) for _ in range(3))
+    k[:, n // 2:, 0] *= 3
+    good = _run(rt, q, k, v, s, n)
+    q2 = q.copy()
+    q2[:, 41], q2[:, 190] = 0, 60
+    got = _run(rt, q2, k, v, s, n)
+    rest = [i for i in range(n) if i not in (41, 190)]
+    assert np.array_equal(got[:, rest], good[:, rest])

@@ -518,13 +518,15 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
 #pragma unroll
       for (int r = 0; r < 16; ++r) mb = fmaxf(mb, s[t][r]);
     mb *= kSDown;
-    // The running max follows only where a score passes it by more than
-    // kSlack (the weights keep that much room below f16's largest value).
+    // A query's running max follows only where one of its scores passes it by
+    // more than kSlack (the weights keep that much room below f16's largest).
     if (__builtin_amdgcn_ballot_w64(mb > m_run + kSlack) != 0) {
       float other;
       mb = xor32_pair(mb, &other);
-      const float m_new = fmaxf(m_run, fmaxf(mb, other));
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 on the first block
+      mb = fmaxf(mb, other);
+      const bool moves = mb > m_run + kSlack;
+      const float m_new = moves ? mb : m_run;
+      const float alpha = moves ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;  // 0 at first
 #pragma unroll
       for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
