@@ -42,9 +42,17 @@
 // instructions 2,478 us.  128-query workgroups there stage twice as often:
 // 1,064 us.
 //
-// Workgroups whose values the split cannot hold (a result that is not finite,
-// or values of V that are all tiny) compute their queries again with F32
-// matrix instructions (attention_tile_f32).
+// A query that the split does not hold (a result that is not finite, or one
+// that is small beside V's columns, kHeldMean) is computed again with F32 matrix
+// instructions by its workgroup, alone: a query's bits depend on its own row and
+// its sequence's K and V only (attention_tile_f32).
+// V of any scale runs at full speed (12 x 866, V x 1e-4: 25 us; judged by one
+// fixed scale 55).  A launch that takes every query again: 12 x 10,392 3.3 ms
+// where K does not fit from the first block on, 3.9 ms where one late value of K
+// or V does not (F32 matrix instructions alone 2.5); 12 x 866 50-53 us (35).
+// What an output may then be off beside F32's rounding: 2^-34 of its V column's
+// largest value in the run's first key block, and 2^-23 of the largest of its
+// query's 64 (each measured against its column).
 #include <cmath>
 
 #include "common.h"
@@ -61,14 +69,18 @@ constexpr int KB = 64;  // keys per block
 constexpr int PITCH = 68;
 constexpr int kSlots = KB * HD / 4;  // float4 of one K (or V) block: 1024
 constexpr float kQScale = 0.125f * 1.44269504088896341f;  // log2(e) / sqrt(64)
-// Scales of the f16 parts (powers of two): K and V by 2^8, Q (with kQScale)
-// by 2^10, the weights by 2^11 with room for a factor 2^4 above the running
-// max.  |k|, |v| of 256 and |q| of 354 no longer fit (those tiles run in F32).
-constexpr float kKvUp = 256.0f, kQUp = 1024.0f, kSDown = 1.0f / 262144.0f;
+// Scales of the f16 parts (powers of two): K by 2^8, Q (with kQScale) by 2^10,
+// the weights by 2^11 with room for a factor 2^4 above the running max.  |k| of
+// 256 and |q| of 354 no longer fit (queries that meet them run in F32).  A
+// column of V is brought to [2^kVBits, 2 x that) by the largest value of the
+// run's first key block; one of 64 to 128 times that no longer fits.
+constexpr float kKUp = 256.0f, kQUp = 1024.0f, kSDown = 1.0f / 262144.0f;
 constexpr float kPBits = 11.0f, kPDown = 1.0f / 2048.0f, kSlack = 4.0f;
-constexpr float kODown = kPDown / kKvUp;
-// The largest |v| from which a run of keys is held (its floor is 2^-33).
-constexpr float kRowMin = 1.0f / 512.0f;
+constexpr int kVBits = 9;
+// A query is held whose largest sum (of 64, over scaled V) reaches both: the
+// floors of V (2^-25 of a scaled value) and of the weights (2^-25 each, of
+// random sign) are then below 2^-24 of that sum.
+constexpr float kHeldMean = 0.5f, kHeldSum = 8192.0f;
 constexpr int kFlush = 8;       // blocks between additions to the running total
 constexpr int kRowBytes = 272;  // LDS pitch of 64 values: 2 parts x 128 bytes + 16
 constexpr int kBufBytes = 2 * KB * kRowBytes;  // a block of K and of V
@@ -111,6 +123,20 @@ __device__ __forceinline__ float group_sum(float v) {
   return v + o;
 }
 
+// Largest |value| over a thread's four and over its row of 16 lanes.
+__device__ __forceinline__ float row16_max(float v) {
+#define VK_ROR(n)                                                                             \
+  v = fmaxf(v, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0x120 | n, 0xf, \
+                                                        0xf, true)));
+  VK_ROR(8) VK_ROR(4) VK_ROR(2) VK_ROR(1)
+#undef VK_ROR
+  return v;
+}
+
+__device__ __forceinline__ float column_max(float a, float b, float c, float d) {
+  return row16_max(fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d))));
+}
+
 __device__ __forceinline__ void split8_plain(const f32x4& x, const f32x4& y, u32x4* p0, u32x4* p1) {
   uint32_t h[4], l[4];
   vks::split2_plain(x[0], x[1], &h[0], &l[0]);
@@ -121,9 +147,9 @@ __device__ __forceinline__ void split8_plain(const f32x4& x, const f32x4& y, u32
   *p1 = u32x4{l[0], l[1], l[2], l[3]};
 }
 
-// The same 64 queries with F32 matrix instructions (four waves of 16 queries;
-// a wave of an eight-wave workgroup past them only helps to stage), for
-// inputs that the split cannot hold.  In the k-permuted fragment order (lane
+// 16 queries a wave with F32 matrix instructions, for those that the split does
+// not hold: bit i of `mask` says whether the wave's query i is stored (a wave
+// without any only helps to stage).  In the k-permuted fragment order (lane
 // group g holds k = 16 b + 4 g + j in component j, MFMA step j takes component
 // j) the A operand of key tile t is the lane's four probabilities of that
 // tile; K is staged as [key][d] and V as [d][key] rows of 68 floats.
@@ -131,7 +157,7 @@ template <bool PART, int kThreads>
 __device__ __forceinline__ void attention_tile_f32(
     float* smem, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, float* __restrict__ out, int sequences, int n, int seq, int qb,
-    int kb_begin, int kb_end, int split, int splits, float* __restrict__ part) {
+    int kb_begin, int kb_end, int split, int splits, float* __restrict__ part, uint32_t mask) {
   constexpr int kPer = kSlots / kThreads;  // staged float4 of K (and of V) per thread
   constexpr int QG = kThreads / 64;
 
@@ -143,7 +169,7 @@ __device__ __forceinline__ void attention_tile_f32(
   float* Ks = smem;
   float* Vt = Ks + KB * PITCH;
   const int q0 = qb + wq * 16;
-  const bool live = wq < 4 && q0 < n;  // uniform over the wave
+  const bool live = mask != 0 && q0 < n;  // uniform over the wave
   const size_t base = static_cast<size_t>(seq) * n * HD;
 
   // Q^T fragments (B operand): query q0 + c16, d = 16 bd + 4 g + j
@@ -223,8 +249,6 @@ __device__ __forceinline__ void attention_tile_f32(
       for (int c = 0; c < 4; ++c) Vt[(d + c) * PITCH + key] = vr[i][c];
     }
     __syncthreads();
-    // a wave whose 16 queries all lie past n only stages (the last query tile
-    // of a sequence whose length is not a multiple of 64)
     if (!live) continue;
 
     // S^T tiles: s[t][r] = score of query q0 + c16 with key k0 + 16t + 4g + r
@@ -319,12 +343,12 @@ __device__ __forceinline__ void attention_tile_f32(
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int qi = q0 + 4 * g + r;
-      if (qi < n) {
+      if (qi < n && ((mask >> (4 * g + r)) & 1)) {
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) po[static_cast<size_t>(qi) * HD + 16 * dt + c16] = o[dt][r];
       }
     }
-    if (g == 0 && q0 + c16 < n)
+    if (g == 0 && q0 + c16 < n && ((mask >> c16) & 1))
       *reinterpret_cast<float2*>(pml + 2 * static_cast<size_t>(q0 + c16)) =
           make_float2(m_run, l_run);
     return;
@@ -335,7 +359,7 @@ __device__ __forceinline__ void attention_tile_f32(
   for (int r = 0; r < 4; ++r) {
     const float lr = __shfl(l_run, 4 * g + r, 64);
     const int qi = q0 + 4 * g + r;
-    if (qi < n) {
+    if (qi < n && ((mask >> (4 * g + r)) & 1)) {
       float* orow = out + base + static_cast<size_t>(qi) * HD + c16;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) orow[16 * dt] = o[dt][r] / lr;
@@ -362,7 +386,8 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
   // with eight waves the first four stage V and the others K
   constexpr bool kShared = QW == 8;
   __shared__ __align__(16) char smem[2 * kBufBytes];
-  __shared__ int flags[QW];
+  __shared__ __align__(16) float vdown[HD];
+  __shared__ uint32_t flags[QW];  // per wave: its queries to compute again
 
   const int tid = threadIdx.x;
   __builtin_assume(tid < kThreads);
@@ -393,7 +418,6 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
     for (int r = 0; r < 16; ++r) o[dt][r] = total[dt][r] = 0.0f;
   float m_run = -INFINITY;  // running max of query q0 + c32 (both halves alike)
   float l_run = 0.0f;       // sum over the keys that this lane holds
-  float vmax = 0.0f;        // largest |v| staged by this thread
 
   // Staging, one block ahead through registers.  K: piece s = 8 floats, key
   // s / 8, d 8 (s % 8).. ; V: 4 keys x 4 d per thread (its lanes in key order:
@@ -426,6 +450,29 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
   };
   load_block(kb_begin);
 
+  // The scale of V's columns 4 d4 .. + 3: the block's largest values (a thread
+  // holds four keys of them, its row of 16 lanes all 64), to the queries' waves
+  // through LDS as 1 / scale.  A column of zeros takes the largest scale: any
+  // value met later is beyond f16, or else too small for any other scale.
+  uint32_t vup = 0;  // the four scales' exponent fields, a byte each
+  if (!upper) {
+    const float m4[4] = {column_max(r0[0].x, r0[1].x, r0[2].x, r0[3].x),
+                         column_max(r0[0].y, r0[1].y, r0[2].y, r0[3].y),
+                         column_max(r0[0].z, r0[1].z, r0[2].z, r0[3].z),
+                         column_max(r0[0].w, r0[1].w, r0[2].w, r0[3].w)};
+    float down[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int b = static_cast<int>(__float_as_uint(m4[c]) >> 23);
+      int e = kVBits + 127 - b;
+      e = b == 255 ? 0 : (m4[c] == 0.0f || e > 126 ? 126 : e);
+      vup |= static_cast<uint32_t>(127 + e) << (8 * c);
+      down[c] = __uint_as_float(static_cast<uint32_t>(127 - e) << 23);
+    }
+    if (quad == 0) *reinterpret_cast<float4*>(vdown + 4 * d4) =
+        make_float4(down[0], down[1], down[2], down[3]);
+  }
+
   // Q^T fragments (B operand): query q0 + c32, d = 16 ks + 8 half + j
   u32x4 qf[4][2];
   {
@@ -448,26 +495,26 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
     for (int i = 0; i < 2; ++i) {
       const float4 x = kr[2 * i], y = kr[2 * i + 1];
       u32x4 p0, p1;
-      split8_plain(f32x4{x.x, x.y, x.z, x.w} * kKvUp, f32x4{y.x, y.y, y.z, y.w} * kKvUp, &p0, &p1);
+      split8_plain(f32x4{x.x, x.y, x.z, x.w} * kKUp, f32x4{y.x, y.y, y.z, y.w} * kKUp, &p0, &p1);
       char* d = k_dst + buf * kBufBytes + 32 * i * kRowBytes;
       *reinterpret_cast<u32x4*>(d) = p0;
       *reinterpret_cast<u32x4*>(d + 128) = p1;
     }
   };
-  auto store_v4 = [&](char* d, float a, float b, float e, float f) {
+  auto store_v4 = [&](char* d, float up, float a, float b, float e, float f) {
     uint32_t p0[2], p1[2];
-    vks::split2_plain(a * kKvUp, b * kKvUp, &p0[0], &p1[0]);
-    vks::split2_plain(e * kKvUp, f * kKvUp, &p0[1], &p1[1]);
+    vks::split2_plain(a * up, b * up, &p0[0], &p1[0]);
+    vks::split2_plain(e * up, f * up, &p0[1], &p1[1]);
     *reinterpret_cast<uint2*>(d) = make_uint2(p0[0], p0[1]);
     *reinterpret_cast<uint2*>(d + 128) = make_uint2(p1[0], p1[1]);
   };
   auto store_v = [&](int buf, const float4 (&vr)[4]) {
-    vmax = fmaxf(vmax, fmaxf(vks::max_abs8(vr[0], vr[1]), vks::max_abs8(vr[2], vr[3])));
     char* d = v_dst + buf * kBufBytes;
-    store_v4(d, vr[0].x, vr[1].x, vr[2].x, vr[3].x);
-    store_v4(d + kRowBytes, vr[0].y, vr[1].y, vr[2].y, vr[3].y);
-    store_v4(d + 2 * kRowBytes, vr[0].z, vr[1].z, vr[2].z, vr[3].z);
-    store_v4(d + 3 * kRowBytes, vr[0].w, vr[1].w, vr[2].w, vr[3].w);
+    auto up = [&](int c) { return __uint_as_float(((vup >> (8 * c)) & 0xffu) << 23); };
+    store_v4(d, up(0), vr[0].x, vr[1].x, vr[2].x, vr[3].x);
+    store_v4(d + kRowBytes, up(1), vr[0].y, vr[1].y, vr[2].y, vr[3].y);
+    store_v4(d + 2 * kRowBytes, up(2), vr[0].z, vr[1].z, vr[2].z, vr[3].z);
+    store_v4(d + 3 * kRowBytes, up(3), vr[0].w, vr[1].w, vr[2].w, vr[3].w);
   };
   auto store_block = [&](int buf) {
     if (upper) {
@@ -587,7 +634,8 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
     const bool more = kb + 1 < kb_end;
     if (more) load_block(kb + 1);
     __builtin_amdgcn_sched_barrier(0);
-    if (live) {
+    // a wave whose queries are all to be taken again only stages
+    if (live && __builtin_amdgcn_ballot_w64(vks::is_finite(l_run)) != 0) {
       if ((kb - kb_begin) % kFlush == kFlush - 1) flush();
       compute(kb, buf);
     }
@@ -597,65 +645,94 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
 
   flush();
 
-  // Did the split hold everything?  (Any value of Q, K or V beyond f16, an
-  // infinity or a NaN makes the sums that it enters NaN or infinite.)
+  // Which queries did the split hold?  Any value of Q, K or V beyond f16, an
+  // infinity or a NaN makes the sums that it enters NaN or infinite; sums that
+  // are all small beside V's columns may show the floors (kHeldMean, kHeldSum).
+  const int qi = q0 + c32;
+  const bool mine = live && qi < n;
   {
     float other;
-    const float mine = xor32_pair(l_run, &other);
-    l_run = mine + other;
+    const float l = xor32_pair(l_run, &other);
+    l_run = l + other;
   }
-  bool odd = live && !vks::is_finite(l_run);
+  bool odd = !vks::is_finite(l_run);
+  float most = 0.0f;
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) odd |= live && !vks::is_finite(total[dt][r]);
-  // V is judged by the largest value of the run: two bits a wave
-  const bool big = vmax >= kRowMin, some = vmax != 0.0f;
-  const int bits = (__builtin_amdgcn_ballot_w64(odd) ? 1 : 0) |
-                   (__builtin_amdgcn_ballot_w64(big) ? 2 : 0) |
-                   (__builtin_amdgcn_ballot_w64(some) ? 4 : 0);
-  if (lane == 0) flags[wave] = bits;
+    for (int r = 0; r < 16; ++r) {
+      odd |= !vks::is_finite(total[dt][r]);
+      most = fmaxf(most, fabsf(total[dt][r]));
+    }
+  {
+    float other;
+    const float m = xor32_pair(most, &other);
+    most = fmaxf(m, other);
+  }
+  const bool small = !(most >= kHeldMean * l_run && most >= kHeldSum);
+  auto queries = [&](bool x) {  // one bit per query of the wave, from either half
+    const uint64_t b = __builtin_amdgcn_ballot_w64(mine && x);
+    return static_cast<uint32_t>(b) | static_cast<uint32_t>(b >> 32);
+  };
+  const uint32_t odd_q = queries(odd), small_q = queries(small);
+  // With every column at the largest scale, V of the run is zeros or has no floor
+  // (2^-25 is then 2^-151 of a value).
+  const bool some =
+      __builtin_amdgcn_ballot_w64(vdown[lane] != __uint_as_float(1u << 23)) != 0;
+  if (lane == 0) flags[wave] = odd_q | (some ? small_q : 0u);
   __syncthreads();
-  int all = 0;
+  
+  uint32_t any = 0;
 #pragma unroll
-  for (int w = 0; w < QW; ++w) all |= flags[w];
-  if (__builtin_expect((all & 1) || (all & 6) == 4, 0)) {
+  for (int w = 0; w < QW; ++w) any |= flags[w];
+  if (mine && ((flags[wave] >> c32) & 1) == 0) {
+    const float* dn = vdown + 4 * half;
+    if constexpr (PART) {
+      // this split's O (rescaled to its own running max), max and sum
+      const size_t rows = static_cast<size_t>(sequences) * n;
+      const size_t row = static_cast<size_t>(split) * rows + static_cast<size_t>(seq) * n + qi;
+      float* po = part + row * HD + 4 * half;
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const f32x4 d = *reinterpret_cast<const f32x4*>(dn + 32 * dt + 8 * r);
+          const f32x4 t = {total[dt][4 * r], total[dt][4 * r + 1], total[dt][4 * r + 2],
+                           total[dt][4 * r + 3]};
+          *reinterpret_cast<f32x4*>(po + 32 * dt + 8 * r) = t * kPDown * d;
+        }
+      if (half == 0)
+        *reinterpret_cast<float2*>(part + static_cast<size_t>(splits) * rows * HD + 2 * row) =
+            make_float2(m_run, l_run * kPDown);
+    } else {
+      // out[query][d] = O / l; both carry the weights' scale, O also V's
+      float* orow = out + base + static_cast<size_t>(qi) * HD + 4 * half;
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const f32x4 d = *reinterpret_cast<const f32x4*>(dn + 32 * dt + 8 * r);
+          const f32x4 t = {total[dt][4 * r] / l_run, total[dt][4 * r + 1] / l_run,
+                           total[dt][4 * r + 2] / l_run, total[dt][4 * r + 3] / l_run};
+          *reinterpret_cast<f32x4*>(orow + 32 * dt + 8 * r) = t * d;
+        }
+    }
+  }
+  if (__builtin_expect(any != 0, 0)) {
+    // 16 queries a wave and pass; the stores are those of the flagged ones
 #pragma unroll 1
-    for (int h = 0; h < QB / 64; ++h) {
+    for (int h = 0; h < 2; ++h) {
+      const int first = 16 * QW * h;  // of the workgroup's queries
+      uint32_t pass = 0;
+      for (int w = first / 32; w < (first + 16 * QW) / 32; ++w) pass |= flags[w];
+      if (pass == 0) continue;
+      const uint32_t mask =
+          (flags[(first + 16 * wave) / 32] >> (16 * (wave & 1))) & 0xffffu;
       __syncthreads();
       attention_tile_f32<PART, kThreads>(reinterpret_cast<float*>(smem), q, k, v, out, sequences,
-                                         n, seq, qb + 64 * h, kb_begin, kb_end, split, splits,
-                                         part);
+                                         n, seq, qb + first, kb_begin, kb_end, split, splits, part,
+                                         mask);
     }
-    return;
-  }
-  const int qi = q0 + c32;
-  if (!live || qi >= n) return;
-  if constexpr (PART) {
-    // this split's O (rescaled to its own running max), max and sum
-    const size_t rows = static_cast<size_t>(sequences) * n;
-    const size_t row = static_cast<size_t>(split) * rows + static_cast<size_t>(seq) * n + qi;
-    float* po = part + row * HD + 4 * half;
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        *reinterpret_cast<f32x4*>(po + 32 * dt + 8 * r) =
-            f32x4{total[dt][4 * r], total[dt][4 * r + 1], total[dt][4 * r + 2], total[dt][4 * r + 3]} * kODown;
-    if (half == 0)
-      *reinterpret_cast<float2*>(part + static_cast<size_t>(splits) * rows * HD + 2 * row) =
-          make_float2(m_run, l_run * kPDown);
-  } else {
-    // out[query][d] = O / l; both carry the weights' scale, O also V's
-    float* orow = out + base + static_cast<size_t>(qi) * HD + 4 * half;
-    const float l = l_run * kKvUp;
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        *reinterpret_cast<f32x4*>(orow + 32 * dt + 8 * r) =
-            f32x4{total[dt][4 * r] / l, total[dt][4 * r + 1] / l, total[dt][4 * r + 2] / l,
-                  total[dt][4 * r + 3] / l};
   }
 }
 
@@ -670,7 +747,7 @@ __global__ __launch_bounds__(256) void attention_short_kernel(const float* __res
                                                               int sequences, int n) {
   __shared__ __align__(16) float smem[2 * KB * PITCH];
   attention_tile_f32<false, 256>(smem, q, k, v, out, sequences, n, blockIdx.x, 0, 0, 1, 0, 1,
-                                 nullptr);
+                                 nullptr, 0xffffu);
 }
 
 // Combines the key splits of the PART form: 16 threads per query row, one
