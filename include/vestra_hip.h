@@ -445,11 +445,13 @@ int vk_linear_run_qkv_hnd_norm_rope_mode_f32(
  * reference: for callers that cannot call hipMalloc (a sequence captured
  * into a HIP graph without an eager run first, serving loops, harnesses that
  * forbid allocation).  The same plan and bits as vk_linear_run_into_f32;
- * split-K partial sums (few rows: an 866-token image's FC2 needs 4 Mi
+ * split-K partial sums (few rows: an 866-token image's FC2 takes 2 Mi
  * floats) go to a static device array of 8 Mi floats (32 MiB, held by each
  * device from the library's load until the process ends) instead of the
- * runtime's work buffer.  A plan needing more than that fails with
- * VK_ERR_UNSUPPORTED and enqueues nothing (e.g. 3,458 rows x 4096 -> 1024).
+ * runtime's work buffer.  A shape for which more than that
+ * must be provided fails with VK_ERR_UNSUPPORTED and enqueues nothing (e.g.
+ * 3,458 rows x 4096 -> 1024, eight slices by the fixed rule that also says
+ * which shapes need an eager call before capture; the plan may take fewer).
  * Every call on one device shares the array: calls on one device that
  * overlap in time (two runtimes' streams) race. */
 int vk_linear_run_into_noalloc_f32(vk_runtime* rt, const vk_linear* lin,

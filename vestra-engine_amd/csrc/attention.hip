@@ -7,7 +7,7 @@
 // splits (split_f16.h), scaled so that the remainders stay normal numbers:
 // one accumulator, the small products first.
 //
-// A workgroup of eight waves (or four, choose_plan) owns 32 queries a wave of
+// A workgroup of eight waves (or four, attention_plan) owns 32 queries a wave of
 // one sequence.  Grids of few tiles split the key blocks of each tile over
 // several workgroups and merge the partial results in a second pass
 // (attention_kernel<true, *>, attention_merge_kernel).  Keys and values stream
@@ -64,8 +64,8 @@ using vks::f32x16;
 using vks::f32x4;
 using vks::u32x4;
 
-constexpr int HD = 64;
-constexpr int KB = 64;  // keys per block
+constexpr int HD = vk::kHeadDim;
+constexpr int KB = vk::kKeyBlock;  // keys per block
 constexpr int PITCH = 68;
 constexpr int kSlots = KB * HD / 4;  // float4 of one K (or V) block: 1024
 constexpr float kQScale = 0.125f * 1.44269504088896341f;  // log2(e) / sqrt(64)
@@ -786,80 +786,6 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __res
       f32x4{o[0] / l, o[1] / l, o[2] / l, o[3] / l};
 }
 
-// Key splits a caller must be ready to provide for: 1 where the shape never
-// splits (it can be captured before any eager call of its kind).  This is the
-// interface's rule, fixed apart from the splits that are taken: 64-query tiles
-// of fewer than two workgroups per CU split to about two (at least two key
-// blocks each, at most 8); fuller grids where a model of 2.2 us per key block of the busiest CU,
-// the partial results' traffic at 5.5 TB/s and 3 us for the merge pass puts a
-// split at least 1% below the unsplit launch.
-int key_splits_to_provide(int cus, size_t sequences, size_t n) {
-  const long long tiles64 = static_cast<long long>(sequences) * ((n + 63) / 64);
-  const int nkb = static_cast<int>((n + KB - 1) / KB);
-  int splits = 1;
-  if (tiles64 < 2LL * cus) {
-    splits = static_cast<int>((2.0 * cus) / static_cast<double>(tiles64) + 0.5);
-    if (splits > nkb / 2) splits = nkb / 2;
-    if (splits > 8) splits = 8;
-    if (splits < 1) splits = 1;
-  } else {
-    constexpr double kBlockUs = 2.2, kBytesPerUs = 5.5e6, kMergeUs = 3.0;
-    const double row_bytes = 4.0 * (HD + 2) * static_cast<double>(sequences * n);
-    const double unsplit = kBlockUs * static_cast<double>((tiles64 + cus - 1) / cus * nkb);
-    double best = unsplit;
-    for (int sp = 2; sp <= 8 && 2 * sp <= nkb; ++sp) {
-      const long long load = (tiles64 * sp + cus - 1) / cus * ((nkb + sp - 1) / sp);
-      const double us = kBlockUs * static_cast<double>(load) +
-                        2.0 * sp * row_bytes / kBytesPerUs + kMergeUs;
-      if (us < best && us < 0.99 * unsplit) {
-        best = us;
-        splits = sp;
-      }
-    }
-  }
-  return splits;
-}
-
-// Waves per workgroup (eight: 256 queries, one workgroup a CU, half the K and V
-// staging per query; four: 128 queries, two a CU) and key splits, from a cost
-// model fitted to sweeps of 12 to 192 sequences of 256 to 10,392 rows: the
-// busiest CU runs ceil(tiles * s / CUs) workgroups of ceil(key blocks / s)
-// blocks each, 2.7 us per block of an eight-wave workgroup, 1.65 of a
-// four-wave one (2.0 where the CU has no second); a split adds its partial
-// results' traffic (s slices of rows x 66 floats written and read back at 5.5
-// TB/s) and the merge pass (about 3 us).  Measured (choice; neighbours): 12 x
-// 10,392 eight waves unsplit 920 us (2 splits 946, four waves 1064); 16 x 3,458
-// eight waves unsplit 150 (2 splits 165, four waves 178); 144 x 866 four waves
-// 104 (eight 124); 12 x 866 four waves in 3 splits 22.1 (unsplit 34.5, eight
-// waves in 4 splits 25.0); 12 x 1,732 eight waves in 3 splits 43 (four waves
-// 47, 2 splits 47).
-struct Plan {
-  int waves, splits;
-};
-
-Plan choose_plan(int cus, size_t sequences, size_t n, int provided) {
-  constexpr double kBytesPerUs = 5.5e6, kMergeUs = 3.0;
-  constexpr double kEightUs = 2.7, kFourUs = 1.65, kFourAloneUs = 2.0;
-  const long long nkb = static_cast<long long>((n + KB - 1) / KB);
-  const double row_bytes = 4.0 * (HD + 2) * static_cast<double>(sequences * n);
-  Plan best{4, 1};
-  double best_us = 0.0;
-  for (const int w : {4, 8}) {
-    const long long tiles = static_cast<long long>(sequences * ((n + 32 * w - 1) / (32 * w)));
-    for (int sp = 1; sp == 1 || (provided > 1 && sp <= 8 && sp <= nkb); ++sp) {
-      const long long load = (tiles * sp + cus - 1) / cus, blocks = (nkb + sp - 1) / sp;
-      double us = static_cast<double>(load * blocks) *
-                  (w == 8 ? kEightUs : (load > 1 ? kFourUs : kFourAloneUs));
-      if (sp > 1) us += 2.0 * sp * row_bytes / kBytesPerUs + kMergeUs;
-      if (best_us == 0.0 || us < best_us) {
-        best = Plan{w, sp};
-        best_us = us;
-      }
-    }
-  }
-  return best;
-}
-
 int check_qkv(const vk_tensor* t, size_t len, const char* what) {
   VK_REQUIRE(t && t->dtype == VK_F32 && t->len == len, "attention: %s must be f32 [%zu] (holds %zu)",
              what, len, t ? t->len : 0);
@@ -894,8 +820,8 @@ int vk_attention_into_f32(vk_runtime* rt, const vk_tensor* q, const vk_tensor* k
   if (len == 0) return VK_OK;
   const int cus = rt->cu_count > 0 ? rt->cu_count : 256;
   const int nkb = static_cast<int>((n + KB - 1) / KB);
-  const int provided = key_splits_to_provide(cus, sequences, n);
-  const Plan plan = choose_plan(cus, sequences, n, provided);
+  const int provided = vk::attention_splits_to_provide(cus, sequences, n);
+  const vk::AttentionPlan plan = vk::attention_plan(cus, sequences, n, provided);
   const int splits = plan.splits, qw = plan.waves;
   const long long tiles = static_cast<long long>(sequences) * ((n + 32 * qw - 1) / (32 * qw));
   const long long blocks = tiles * splits;

@@ -13,6 +13,7 @@
 #include <tuple>
 #include <vector>
 
+#include "plans.h"
 #include "vestra_hip.h"
 
 // ---------------------------------------------------------------------------
@@ -270,10 +271,6 @@ enum LinearEpilogue {
 };
 }  // namespace linear_epilogue
 
-constexpr int kSplitK = 32;  // k of one stage of the wide kernel
-// Most floats of split-K partial sums: the allocation-free entry point's
-// scratch, so a plan that splits always fits it.
-constexpr long long kMaxPartialFloats = 8LL << 20;
 // The wide-tile linear (128 x 256 to 64 x 64 tiles, split-K for few rows) for
 // K % 4 == 0 and a 16-byte aligned x (linear.hip); the head-major layouts of
 // LinearArgs need it.

@@ -185,10 +185,9 @@ __device__ __forceinline__ float4 qk_head_row(const LinearArgs& g, float4 v, int
       v, l, gm, bt, py, px, g.qkn.table, g.qkn.table_max, g.qkn.eps);
 }
 
-// Most split-K slices a sum pass reads (choose_plan and slices_to_provide).
-// The sum passes are instantiated for split-count buckets SPB of 2, 4 and 8
-// (split_bucket).
-constexpr int kMaxSplits = 8;
+// The sum passes are instantiated for split-count buckets SPB of 2, 4 and 8 (a
+// plan takes at most kMaxSplits).
+static_assert(vk::kMaxSplits <= 8, "split_bucket");
 constexpr int split_bucket(int splits) { return splits <= 2 ? 2 : (splits <= 4 ? 4 : 8); }
 
 // The NV float4 at offsets e[i] of every split's slice (splits <= SPB),
@@ -858,112 +857,8 @@ namespace vk {
 
 namespace {
 
-struct Plan {
-  int tm, tn;
-  int splits;
-  long long tiles;
-};
-
-long long tile_count(int tm, int tn, int M, int N) {
-  return static_cast<long long>((M + tm - 1) / tm) * static_cast<long long>((N + tn - 1) / tn);
-}
-
-// Partial slices a caller must be ready to provide for: 1 where the shape
-// never splits (it can be captured before any eager call of its kind), else
-// the count that the allocation-free entry point's scratch is held against.
-// This is the interface's rule, fixed apart from what a plan takes (a plan
-// never takes more floats than this count, or kMaxPartialFloats): the
-// cheapest of 128 x 128, 64 x 128 and 64 x 64 tiles in runs of 64-wide K
-// chunks, at 5.5 us per chunk of the busiest CU's 128 x 128 tiles (0.6 and
-// 0.28 of that for the others) plus the partial sums' traffic at 5.5 TB/s
-// and 2 us for the sum pass; on ties the larger tile, then the smaller count.
-int slices_to_provide(long long cus, int M, int N, int K) {
-  constexpr double kChunkUs = 5.5, kBytesPerUs = 5.5e6, kSumLaunchUs = 2.0;
-  struct Shape {
-    int tm, tn;
-    double cost;
-  };
-  constexpr Shape kShapes[] = {{128, 128, 1.0}, {64, 128, 0.6}, {64, 64, 0.28}};
-  const int nch = (K + 63) / 64;
-  const long long mn = static_cast<long long>(M) * N;
-  int best = 0;
-  double best_us = 0.0;
-  for (const Shape& sh : kShapes) {
-    const long long tiles = tile_count(sh.tm, sh.tn, M, N);
-    for (int sp = 1; sp == 1 || (sp <= kMaxSplits && 2 * sp <= nch && sp * mn <= (1LL << 26));
-         ++sp) {
-      const long long load = (tiles * sp + cus - 1) / cus * ((nch + sp - 1) / sp);
-      double us = kChunkUs * sh.cost * static_cast<double>(load);
-      if (sp > 1) us += 8.0 * static_cast<double>(sp * mn) / kBytesPerUs + kSumLaunchUs;
-      if (best == 0 || us < best_us) {
-        best = sp;
-        best_us = us;
-      }
-    }
-  }
-  return best;
-}
-
-// Tile shape and split count, from a cost model fitted to plan sweeps of
-// the ViT-B and ViT-L projections at 100 to 10,392 rows.  Workgroups are
-// dealt round-robin to the CUs, so the busiest CU runs ceil(tiles * s / CUs)
-// workgroups of up to ceil(stages / s) 32-wide K stages each: 1.3 us per stage
-// of a 128 x 256 tile (and 3 us per tile that nothing else on the CU covers),
-// 0.85 of a 128 x 128, 0.43 of a 64 x 128 and 0.26 of a 64 x 64 one; of the
-// latter three, a CU with one workgroup has nothing to cover its waits and
-// counts 1.3.  A split adds its partial sums (s x M x N floats written, then
-// read by the sum pass, at about 5.5 TB/s) and the sum pass's launch (about 2
-// us).  The cheapest plan wins; on ties the first shape, then the smaller
-// count.  At least four stages per
-// split; where the shape may split, at most kMaxStages of them (a run's
-// rounding grows with its length: K = 4096, 4.1e-7 of the 64-bit result
-// unsplit, 3.0e-7 in two).  Measured (model's choice; neighbours): 866 x 768 ->
-// 2304, 64 x 64 17.2 us (64 x 128 18.2, 128 x 128 29); 866 x 3072 -> 768, 64 x
-// 64 x 3 24.4 (unsplit 35, 64 x 128 x 6 24.3); 1500 x 768 -> 2304, 64 x 128 24.3
-// (64 x 64 27, 128 x 128 30); 3458 x 4096 -> 1024, 128 x 256 x 2 90 (64 x 128
-// 97, 128 x 128 x 2 99); 10,392 x 3072 -> 768, 128 x 256 127 (128 x 128 136, 64
-// x 128 154).
-constexpr int kMaxStages = 96;
-
-Plan choose_plan(long long cus, int M, int N, int K, int provided) {
-  constexpr double kBytesPerUs = 5.5e6, kSumLaunchUs = 2.0, kAlone = 1.3;
-  // tile shape, us of one of its K stages, of one of its tiles, and the load
-  // that a lone workgroup counts
-  struct Shape {
-    int tm, tn;
-    double us, tile_us, alone;
-  };
-  constexpr Shape kShapes[] = {{128, 256, 1.3, 3.0, 1.0},
-                               {128, 128, 0.85, 0.0, kAlone},
-                               {64, 128, 0.43, 0.0, kAlone},
-                               {64, 64, 0.26, 0.0, kAlone}};
-  const int nch = (K + KC - 1) / KC;
-  const long long mn = static_cast<long long>(M) * N;
-  const auto may = [&](int sp) {
-    return sp == 1 || (provided > 1 && sp <= kMaxSplits && 4 * sp <= nch &&
-                       (sp <= provided || sp * mn <= kMaxPartialFloats));
-  };
-  Plan best{0, 0, 1, 0};
-  double best_us = 0.0;
-  for (const Shape& sh : kShapes) {
-    const long long tiles = tile_count(sh.tm, sh.tn, M, N);
-    for (int sp = 1; may(sp); ++sp) {
-      const int stages = (nch + sp - 1) / sp;
-      if (stages > kMaxStages && may(sp + 1)) continue;
-      const double load = static_cast<double>((tiles * sp + cus - 1) / cus);
-      double us = (sh.us * stages + sh.tile_us) * (load > 1.0 ? load : sh.alone);
-      if (sp > 1) us += 8.0 * static_cast<double>(sp * mn) / kBytesPerUs + kSumLaunchUs;
-      if (best.tm == 0 || us < best_us) {
-        best = Plan{sh.tm, sh.tn, sp, tiles};
-        best_us = us;
-      }
-    }
-  }
-  return best;
-}
-
 template <int EPI, int LAY, int QKN, int NP>
-void launch_tiles(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 grid) {
+void launch_tiles(vk_runtime* rt, const LinearArgs& g, const LinearPlan& plan, dim3 grid) {
   if (plan.tn == 256)
     hipLaunchKernelGGL((linear_wide_kernel<EPI, LAY, QKN, 128, 256, 1, NP>), grid, dim3(512), 0,
                        rt->stream, g);
@@ -979,7 +874,7 @@ void launch_tiles(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 gr
 }
 
 template <int EPI, int LAY, int QKN = 0>
-void launch_pair(vk_runtime* rt, const LinearArgs& g, const Plan& plan, dim3 grid,
+void launch_pair(vk_runtime* rt, const LinearArgs& g, const LinearPlan& plan, dim3 grid,
                  bool sum_pass = true) {
   if (g.wparts == 1)
     launch_tiles<EPI, LAY, QKN, 1>(rt, g, plan, grid);
@@ -1151,8 +1046,8 @@ int launch_linear_wide(vk_runtime* rt, const LinearArgs& g0, int epi, float* par
   // plan, and the plan on (M, N, K) alone, so every layout and epilogue of one
   // shape gives the same bits.
   const long long cus = rt->cu_count > 0 ? rt->cu_count : 256;
-  const int provided = slices_to_provide(cus, g.M, g.N, g.K);
-  const Plan plan = choose_plan(cus, g.M, g.N, g.K, provided);
+  const int provided = linear_slices_to_provide(cus, g.M, g.N, g.K);
+  const LinearPlan plan = linear_plan(cus, g.M, g.N, g.K, provided);
   g.splits = plan.splits;
   g.partial = nullptr;
   VK_UNSUPPORTED_IF(plan.tiles * g.splits > 0x7fffffffLL, "linear: %lld tiles", plan.tiles);
@@ -1162,14 +1057,14 @@ int launch_linear_wide(vk_runtime* rt, const LinearArgs& g0, int epi, float* par
   if (provided > 1) {
     VK_REQUIRE(g.N % 4 == 0, "linear: split-K needs out_features % 4 == 0");
     const size_t mn = static_cast<size_t>(g.M) * g.N;
+    const int most = provided > g.splits ? provided : g.splits;
     if (partial) {
-      VK_UNSUPPORTED_IF(provided * mn > partial_floats,
+      VK_UNSUPPORTED_IF(most * mn > partial_floats,
                         "linear (M=%d, N=%d, K=%d): %d split-K slices need %zu floats of "
                         "scratch, more than the %zu available",
-                        g.M, g.N, g.K, provided, provided * mn, partial_floats);
+                        g.M, g.N, g.K, most, most * mn, partial_floats);
       g.partial = partial;
     } else {
-      const size_t most = provided > g.splits ? provided : g.splits;
       VK_TRY(vk::ensure_work(rt, most * mn, "linear (split-K)"));
       g.partial = rt->work;
     }

@@ -531,7 +531,9 @@ int vk_linear_run_hnd_residual_f32(vk_runtime* rt, const vk_linear* lin, const v
 // pass reads it, so nothing needs clearing, but calls that overlap on one
 // device (two runtimes' streams at once) race on it.
 // ---------------------------------------------------------------------------
-constexpr size_t kScratchFloats = size_t{8} << 20;  // 32 MiB per device
+// 32 MiB per device; a plan that splits takes no more than this (linear_plan), and
+// the launch compares what it takes with it.
+constexpr size_t kScratchFloats = static_cast<size_t>(vk::kMaxPartialFloats);
 
 static __device__ __align__(256) float scratch[kScratchFloats];
 
