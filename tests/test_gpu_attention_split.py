@@ -21,9 +21,15 @@ vh = pytest.importorskip("vestra_hip")
 
 FLOOR = 2.0 ** -33
 
-# sequences, rows: four waves unsplit, eight waves unsplit, four waves in three and
-# in eight key splits, eight waves in three
-FORMS = [(250, 300), (40, 800), (12, 866), (2, 1000), (12, 1732)]
+# sequences and rows of one shape for each kernel form, and its (waves, key splits) on
+# 256 compute units (test_plans.py holds the tables to the rules)
+FORM_OF = {(250, 300): (4, 1), (40, 800): (8, 1), (12, 866): (4, 3), (2, 1000): (4, 8),
+           (12, 1732): (8, 3)}
+FORMS = list(FORM_OF)
+# one block and one past it, 128- and 256-query tiles and one past each
+SIZE_FORM = {(2, 63): (4, 1), (3, 66): (4, 1), (2, 127): (4, 1), (2, 128): (4, 1),
+             (12, 190): (4, 1), (2, 513): (4, 5), (130, 129): (8, 1), (250, 257): (4, 1),
+             (250, 320): (4, 1), (40, 800): (8, 1), (12, 1740): (8, 3)}
 
 
 def _assert_close(got, q, k, v, label, channel_floor=FLOOR):
@@ -45,11 +51,7 @@ def _some(s):
     return range(0, s, max(1, s // 3))
 
 
-# one block and one past it, 128- and 256-query tiles and one past each, without
-# key splits (four waves: 2 x 127, 12 x 190, 250 x 257; eight: 130 x 129) and with
-# (2 x 513: five of four waves; 12 x 1740: three of eight)
-@pytest.mark.parametrize("s,n", [(2, 63), (3, 66), (2, 127), (2, 128), (12, 190), (2, 513),
-                                 (130, 129), (250, 257), (250, 320), (40, 800), (12, 1740)])
+@pytest.mark.parametrize("s,n", list(SIZE_FORM))
 def test_sizes(rt, rng, s, n):
     q, k, v = (normals(rng, s, n, 64) for _ in range(3))
     _check(rt, q, k, v, f"n={n}", _some(s))

@@ -37,13 +37,17 @@ def _check(got, x, w, b, label, terms=None):
     assert not bad.any(), f"{label}: {int(bad.sum())} off, worst {np.max(np.abs(got - ref) / tol)}"
 
 
-# 64 x 64 tiles (2 stages a barrier: odd counts, tails; 130 x 3072 -> 132 in eight
-# splits), 64 x 128, 128 x 128 and 128 x 256 (with rows and columns past a tile; in
-# four splits), rows and columns one past a tile, K below one stage
-@pytest.mark.parametrize("m,k,n", [(1, 4, 4), (63, 28, 60), (65, 96, 68), (64, 100, 64),
-                                   (130, 3072, 132), (1500, 160, 2304), (10392, 64, 768),
-                                   (4097, 132, 1540), (4000, 1024, 1028), (10392, 768, 768),
-                                   (2600, 3072, 772)])
+# tails of rows, columns and K on every tile; K below one stage; odd counts of 32 k
+# on tiles of two a barrier
+SHAPE_FORM = {(1, 4, 4): (64, 64, 1), (63, 28, 60): (64, 64, 1), (65, 96, 68): (64, 64, 1),
+              (64, 100, 64): (64, 64, 1), (130, 3072, 132): (64, 64, 8),
+              (1500, 160, 2304): (64, 128, 1), (4000, 1024, 1028): (64, 128, 1),
+              (10392, 64, 768): (128, 128, 1), (4097, 132, 1540): (128, 128, 1),
+              (10392, 768, 768): (128, 256, 1), (10300, 804, 764): (128, 256, 1),
+              (2600, 3072, 772): (128, 256, 3)}
+
+
+@pytest.mark.parametrize("m,k,n", list(SHAPE_FORM))
 def test_shapes(rt, rng, m, k, n):
     x, w, b = normals(rng, m, k), normals(rng, k, n, scale=0.02), normals(rng, n, scale=0.02)
     _check(_linear(rt, x, w, b), x, w, b, f"{m}x{k}->{n}")
@@ -111,10 +115,12 @@ def test_f16_stored_weights_are_the_f32_preparation(rt, rng, m, k, n, wide_range
     _check(out.numpy().reshape(m, n), x, w.astype(np.float32), b, "f16 weights")
 
 
-# one tile shape each (64 x 64 in six splits, 64 x 128, 128 x 128, 128 x 256, and
-# 128 x 256 in four splits)
-FORMS = [(130, 768, 192), (1500, 768, 2304), (10392, 128, 768), (10392, 768, 768),
-         (2600, 3072, 768)]
+# rows, k, columns of one shape for each tile, and its (rows, columns, splits) on 256
+# compute units (test_plans.py holds the table to the rules)
+FORM_OF = {(130, 768, 192): (64, 64, 6), (1500, 768, 2304): (64, 128, 1),
+           (10392, 128, 768): (128, 128, 1), (10392, 768, 768): (128, 256, 1),
+           (2600, 3072, 768): (128, 256, 4)}
+FORMS = list(FORM_OF)
 
 
 @pytest.mark.parametrize("m,k,n", FORMS)

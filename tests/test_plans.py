@@ -50,3 +50,19 @@ def test_the_fixed_scratch_is_the_plans_limit():
     assert re.search(r"kScratchFloats = static_cast<size_t>\(vk::kMaxPartialFloats\);", src)
     launch = open(os.path.join(plans._CSRC, "linear.hip")).read()
     assert "VK_UNSUPPORTED_IF(most * mn > partial_floats" in launch
+
+
+def test_the_gpu_tests_reach_the_forms_they_name():
+    """Shapes of the GPU tests against the rules: a change of their constants that
+    moves a shape to another form is seen here."""
+    attention = pytest.importorskip("test_gpu_attention_split")
+    linear = pytest.importorskip("test_gpu_linear_split")
+    for table in (linear.FORM_OF, linear.SHAPE_FORM):
+        for (m, k, n), form in table.items():
+            assert tuple(plans.linear_form(m, k, n)[:3]) == form, (m, k, n)
+    assert {f[:2] for f in linear.FORM_OF.values()} == {(64, 64), (64, 128), (128, 128), (128, 256)}
+    for table in (attention.FORM_OF, attention.SIZE_FORM):
+        for (s, n), form in table.items():
+            assert tuple(plans.attention_form(s, n)[:2]) == form, (s, n)
+    assert {(w, sp > 1) for w, sp in attention.FORM_OF.values()} == {(4, False), (4, True),
+                                                                     (8, False), (8, True)}
