@@ -67,11 +67,11 @@ struct vk_linear {
   size_t k_pitch = 0;          // in_features rounded up to 16
   float* weight_nk = nullptr;  // [out, k_pitch], input dimension contiguous
   // The rows as f16 parts in the wide linear's fragment order, each row
-  // scaled by 2^weight_exp (split_weights), for in_features % 4 == 0.
+  // scaled by 2^weight_col.x (split_weights), for in_features % 4 == 0.
   void* weight_split = nullptr;
-  // In its allocation: the rows' exponents [out], and running counts of what
-  // the values are, [1 + stages][out].
-  int* weight_exp = nullptr;
+  // In its allocation: the rows' exponents and sums [out], and running counts of
+  // what the values are, [1 + stages][out].
+  int2* weight_col = nullptr;
   uint2* weight_stat = nullptr;
   int weight_parts = 0;        // 1 where every second part is zero (f16 values)
   // For a 3x14x14 patch filter (in_features 588) only: the same rows with
@@ -177,7 +177,7 @@ void noalloc_setup(int device);
 // (c, ky, kx) -> (ky, kx, c) of an HWC image's patch, zero-padded to 592, on
 // the runtime's stream.  Any other linear: nothing.
 int prepare_patch_filter(vk_runtime* rt, vk_linear* lin);
-// Allocates and fills lin->weight_split and weight_exp from lin->weight_nk (whose writes have
+// Allocates and fills lin->weight_split and what goes with it from lin->weight_nk (whose writes have
 // finished); the default stream, waited for.  in_features % 4 != 0: nothing.
 // f16_values: the weights were stored as f16.
 int split_weights(vk_linear* lin, bool f16_values);
@@ -226,7 +226,7 @@ struct LinearArgs {
   const float* x;     // [M, K]
   const float* wnk;   // [N, Kp], K contiguous, zero beyond K
   const void* wsplit; // its f16 parts (vk_linear::weight_split) and
-  const int* wexp;    // their rows' exponents and counts, linear.hip only
+  const int2* wcol;   // their rows' exponents and counts, linear.hip only
   const uint2* wstat;
   int wparts;         // parts of a weight (vk_linear::weight_parts)
   const float* bias;  // [N]

@@ -62,21 +62,23 @@
 //    those with a value below 2^-13 (tiny), a column its groups of weights all of
 //    at least 8 (dense) and its weights below 2^-13 that their parts do not hold
 //    exactly (tiny).  Then
-//      the floor's share of a sum   <= 2^-24 (4 tiny_row + 16 tiny_col),
+//      the floor's share of a sum   <= 2^-24 need,
+//        need = min(4 tiny_row, 2^-12 sum |w|) + 16 tiny_col,
 //      the sum of its |terms|  s    >= 8 (big + dense - G)  and  >= |sum|,
-//    the first bound because at least big + dense - G groups hold a value of at
-//    least 1 whose weight is at least 8.  Taken again unless one of the two
-//    reaches 4 tiny_row + 16 tiny_col: the floor then stays below 2^-24 s;
+//    the former because at least big + dense - G groups hold a value of at least 1
+//    whose weight is at least 8.  Taken again unless one of the two reaches
+//    `need`: the floor then stays below 2^-24 s;
 //  * a sum of few terms, which F32 adds with next to no rounding (a one-hot
 //    column copies): fewer than 8 groups of the row reach 1, or of the column 8.
 // Ordinary rows (layer-normalised, GELU outputs, attention outputs) and dense
 // columns pass as a whole; then an output costs only the test that it is finite.
-// The scale and the counts take 0.5 to 0.9 us of a launch of one image (866 x 768
-// -> 2304 18.2 -> 19.2 us) and 1 to 3% of the large ones.  Rows of any scale up to
-// f32's run at that speed (x 1e-6: 20.6 us; judged by a fixed scale and taken
-// again tile by tile 69).  A launch that takes every output again (NaN
-// throughout; eight decades of sizes in every row) costs about 1.8 times one on
-// F32 matrix instructions alone: 10,392 x 768 -> 3072 740 us against 386.
+// The scale and the counts take 0.5 to 1.1 us of a launch of one image (866 x 768
+// -> 2304 17.1 -> 18.0 us, projection 12.3 -> 12.8) and 2 to 4% of the large ones
+// (10,392 x 768 -> 3072 154 -> 158).  Rows of any scale run at that speed (x 1e-6:
+// 20.5 us a call; judged by one fixed scale and taken again tile by tile 69), and
+// so do eight decades of sizes in every row at 866 rows (22.8).  A launch that
+// takes every output again (NaN throughout) costs about 1.8 times one on F32 matrix
+// instructions alone: 10,392 x 3072 -> 768 684 us against 375.
 //
 // Tiles are numbered XCD-major in groups of at most 1,024 rows (tile_of): the
 // workgroups an XCD holds at one time then share both a slice of A and one
@@ -100,12 +102,12 @@ constexpr int waves_for(int tn) { return tn == 256 ? 8 : 4; }
 constexpr float kTiny = 1.0f / 8192.0f, kXBig = 1.0f, kWBig = 8.0f;
 // A row's typical value is brought to [2^kRowBits, 2 x that), its largest one
 // (of those looked at) below 2^(kRowMaxBits + 1).
-constexpr int kRowBits = 6, kRowMaxBits = 13;
+constexpr int kRowBits = 6, kRowMaxBits = 9;
 constexpr int kFewGroups = 8;      // sums of fewer groups than this are F32 sums
 // The linears of the split: at least kFewGroups groups, counts of 16 bits.
 constexpr int kMinSplitK = 8 * kFewGroups, kMaxSplitK = 1 << 18;
 constexpr int kZeroColumn = 1 << 20;  // exponent of a column of zeros
-constexpr int kZeroRow = 0xffff;      // count of a row of zeros
+constexpr int kZeroRowExp = 126;      // and of a row without a value in the sample
 constexpr int kRowBytes = 144;     // LDS pitch of a row of A: 2 parts x 64 bytes + 16
 constexpr int kXsPitch = 68;       // f32 pitch of the Q/K epilogue's rows
 static_assert(kRowBytes % 16 == 0 && (kRowBytes / 16) % 2 == 1 && kRowBytes >= 4 * KC, "pitch");
@@ -232,6 +234,10 @@ __device__ __forceinline__ void tile_of(int t, int gmt, int gnt, int splits, int
   *split = rest / gnt;
 }
 
+__device__ __forceinline__ float max_abs4(const float4& x) {
+  return fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
+}
+
 // Largest value and sum over the four lanes 4 i .. 4 i + 3 (a row's pieces).
 __device__ __forceinline__ uint32_t quad_other(uint32_t v, int step) {
   const int x = static_cast<int>(v);  // quad_perm [1, 0, 3, 2] and [2, 3, 0, 1]
@@ -255,15 +261,13 @@ __device__ __forceinline__ float quad_max(float v) {
 // KS: stages of 32 k per barrier (2 for the 64-row tiles, whose 12 or 24
 // MFMAs a wave and stage are too few to cover a load's latency).
 // What a column's weights are in stages [c_begin, c_end): groups of 8 k all of
-// at least kWBig, groups that reach it, weights with a floor (split_weights).
+// at least kWBig, groups that reach it, weights with a floor (split_weights), from
+// the running counts `a` before c_begin and `b` before c_end.
 struct ColumnRun {
   int dense, any, tiny;
 };
 
-__device__ __forceinline__ ColumnRun column_run(const LinearArgs& g, int col, int c_begin,
-                                                int c_end) {
-  const uint2 a = g.wstat[static_cast<size_t>(c_begin) * g.N + col];
-  const uint2 b = g.wstat[static_cast<size_t>(c_end) * g.N + col];
+__device__ __forceinline__ ColumnRun column_run(const uint2& a, const uint2& b) {
   return ColumnRun{static_cast<int>((b.x - a.x) & 0xffffu),
                    static_cast<int>((b.x >> 16) - (a.x >> 16)) & 0xffff,
                    static_cast<int>(b.y - a.y)};
@@ -342,11 +346,10 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
             a_rsrc, 8 * piece + 4 * h < left ? a_off[i] + 16u * h : 0xfffffff0u, base);
     }
   };
-  // Per row of the thread's slots: its scale, the groups counted, the bits of any
-  // first part.
+  // Per row of the thread's slots: its scale and the groups counted.
   constexpr int kVR = kVA / KS;
   float rscale[kVR];
-  uint32_t rbig[kVR], rtiny[kVR], rany[kVR];
+  uint32_t rbig[kVR], rtiny[kVR];
   auto store_a = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < kVA; ++i) {
@@ -356,7 +359,6 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
       rtiny[rr] += vks::min_abs8(x, y) < kTiny;
       u32x4 p0, p1;
       vks::split8(x, y, &p0, &p1);
-      rany[rr] |= p0[0] | p0[1] | p0[2] | p0[3];
       char* d = smem + buf * kBufBytes + slot_stage(i) * kStageBytes + slot_row(i) * kRowBytes +
                 16 * piece;
       *reinterpret_cast<u32x4*>(d) = p0;
@@ -430,40 +432,45 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   const int groups = 4 * (c_end - c_begin);
   auto col_of = [&](int u) { return n0 + wave * WN + u * 16 + (lane & 15); };
   int cexp[NU];
-  ColumnRun cr[NU];
+  float cfloor[NU];
+  uint2 cr0[NU], cr1[NU];  // read here, and looked at after the loop
   int ch = split_k ? c_begin : c_end;
   if (split_k) {
     load_a(c_begin, ra);
-    float4 rm[kVA][2];  // the run's middle, for the scale
-    load_a((c_begin + c_end) >> 1, rm);
+    float4 rm[kVR];  // of the run's middle, for the scale
+    const int mid = (c_begin + c_end) >> 1;
+#pragma unroll
+    for (int i = 0; i < kVR; ++i)
+      rm[i] = vkd::buffer_load4(a_rsrc, 8 * piece < g.K - mid * KC ? a_off[i] : 0xfffffff0u,
+                                a_chunk(mid));
     load_b(c_begin, b0);
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int col = col_of(u) < g.N ? col_of(u) : g.N - 1;
-      cexp[u] = g.wexp[col];
-      cr[u] = column_run(g, col, c_begin, c_end);
+      const int2 c = g.wcol[col];
+      cexp[u] = c.x;
+      cfloor[u] = __int_as_float(c.y);
+      cr0[u] = g.wstat[static_cast<size_t>(c_begin) * g.N + col];
+      cr1[u] = g.wstat[static_cast<size_t>(c_end) * g.N + col];
     }
+    // every load issued before the first is waited for
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < kVR; ++i) {
-      float m = 0.0f, t = 0.0f;
-#pragma unroll
-      for (int j = i; j < kVA; j += kVR) {
-        const float first = vks::max_abs8(ra[j][0], ra[j][1]);
-        const float mid = vks::max_abs8(rm[j][0], rm[j][1]);
-        m = fmaxf(m, fmaxf(first, mid));
-        t = fmaxf(t, fminf(first, mid));
-      }
-      m = quad_max(m);  // the four pieces of a row are adjacent lanes
-      t = quad_max(t);
+      // the pieces of the first stage and half of those of the middle one; the
+      // typical size is the lesser of the two, of the row's best piece
+      const float first = vks::max_abs8(ra[i][0], ra[i][1]), middle = max_abs4(rm[i]);
+      const float m = quad_max(fmaxf(first, middle)), t = quad_max(fminf(first, middle));
       // values in [2^(b - 127), 2^(b - 126)).  No value seen: the largest scale, by
-      // which every other f32 has a first part that is not 0.
+      // which any value met later is beyond f16, or has no floor (a row of zeros
+      // is held).
       const int bm = static_cast<int>(__float_as_uint(m) >> 23);
       const int bt = t > 0.0f ? static_cast<int>(__float_as_uint(t) >> 23) : bm;
       int e = kRowBits + 127 - bt;
       e = e < kRowMaxBits + 127 - bm ? e : kRowMaxBits + 127 - bm;
       e = bm == 255 ? 0 : (m == 0.0f || e > 126 ? 126 : e);
       rscale[i] = __uint_as_float(static_cast<uint32_t>(127 + e) << 23);
-      rbig[i] = rtiny[i] = rany[i] = 0;
+      rbig[i] = rtiny[i] = 0;
     }
     store_a(0);
     load_a(ch + KS, ra);
@@ -494,12 +501,15 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   int* row_cnt = row_exp + TM;
   int* flags = row_cnt + TM;  // one per wave: a row that is not plain
   bool look = !split_k;
+  ColumnRun cr[NU];
   if (split_k) {
 #pragma unroll
-    for (int u = 0; u < NU; ++u)
+    for (int u = 0; u < NU; ++u) {
+      cr[u] = column_run(cr0[u], cr1[u]);
       look |= (cexp[u] != kZeroColumn) &
               ((cr[u].any < kFewGroups) |
                (8 * (cr[u].dense - groups) - 16 * cr[u].tiny < -6 * groups));
+    }
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -517,11 +527,11 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
       const int tiny = static_cast<int>(
           quad_sum(rtiny[i] - ((c_end - c_begin) % KS != 0 ? 1u : 0u)));
       const int big = static_cast<int>(quad_sum(rbig[i]));
-      const uint32_t any = quad_sum(rany[i] & 0x7fff7fffu ? 1u : 0u);
-      plain_rows &= any == 0 || (big >= kFewGroups && 8 * big - 4 * tiny >= 6 * groups);
+      const int e = static_cast<int>(__float_as_uint(rscale[i]) >> 23) - 127;
+      plain_rows &= e == kZeroRowExp || (big >= kFewGroups && 8 * big - 4 * tiny >= 6 * groups);
       if (piece == 0) {
-        row_exp[slot_row(i)] = static_cast<int>(__float_as_uint(rscale[i]) >> 23) - 127;
-        row_cnt[slot_row(i)] = any == 0 ? kZeroRow : tiny << 16 | big;
+        row_exp[slot_row(i)] = e;
+        row_cnt[slot_row(i)] = tiny << 16 | big;
       }
     }
     const bool rows_look = __builtin_amdgcn_ballot_w64(!plain_rows) != 0;
@@ -572,11 +582,12 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
           for (int r = 0; r < 4; ++r) {
             const float v = acc[t][u][r];
             const int big = c[r] & 0xffff, tiny = (c[r] >> 16) & 0xffff;
-            const int need = 4 * tiny + 16 * cr[u].tiny;
+            const float need = fminf(static_cast<float>(4 * tiny), cfloor[u]) +
+                               static_cast<float>(16 * cr[u].tiny);
             const bool held =
-                c[r] == kZeroRow || cexp[u] == kZeroColumn ||
+                e[r] == kZeroRowExp || cexp[u] == kZeroColumn ||
                 (big >= kFewGroups && cr[u].any >= kFewGroups &&
-                 (8 * (big + cr[u].dense - groups) >= need || fabsf(v) >= static_cast<float>(need)));
+                 fmaxf(static_cast<float>(8 * (big + cr[u].dense - groups)), fabsf(v)) >= need);
             if (!held || !vks::is_finite(v)) again[i] |= 1u << (4 * u + r);
             acc[t][u][r] = __builtin_amdgcn_ldexpf(v, -e[r] - cexp[u]);
           }
@@ -902,13 +913,14 @@ void launch_pair(vk_runtime* rt, const LinearArgs& g, const LinearPlan& plan, di
 
 }  // namespace
 
-// Exponent of each weight column for the split: wexp[n] = e brings the
-// column's largest |w| to 2^e |w| in [2^10, 2^11), so that every value down to
-// 2^-24 of it has both parts (kZeroColumn for a column of zeros).
-__global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __restrict__ wnk,
-                                                              int* __restrict__ wexp, int N,
-                                                              int Kp) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) wexp[N] = 0;  // split_weights_kernel's flag
+// Per weight column: the split's exponent e, which brings the column's largest
+// |w| to 2^e |w| in [2^10, 2^11), so that every value down to 2^-24 of it has both
+// parts (kZeroColumn for a column of zeros); and the floor's share of a sum whose
+// other factors are all tiny, 2^24 x 2^-36 x the sum of the scaled |w|.
+__global__ __launch_bounds__(256) void weight_column_kernel(const float* __restrict__ wnk,
+                                                            int2* __restrict__ wcol, int N,
+                                                            int Kp) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) wcol[N].x = 0;  // split_weights_kernel's flag
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= N) return;
   uint32_t m = 0;
@@ -923,10 +935,19 @@ __global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __res
   }
   int e = 0;
   if (m) (void)frexpf(__uint_as_float(m), &e);  // m in [2^(e-1), 2^e)
-  if (lane == 0) wexp[row] = m ? 11 - e : kZeroColumn;
+  e = m ? 11 - e : kZeroColumn;
+  float sum = 0.0f;
+  for (int k = lane; k < Kp; k += 64) {
+    const float w = fabsf(ldexpf(wnk[static_cast<size_t>(row) * Kp + k], e));
+    if (vks::is_finite(w)) sum += w;
+  }
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) sum += __shfl_xor(sum, s, 64);
+  // a little more than the sum, for its rounding
+  if (lane == 0) wcol[row] = make_int2(e, __float_as_int(sum * (1.01f / 4096.0f)));
 }
 
-// The f16 parts of the scaled rows 2^wexp[n] wnk[n] of [N, Kp] in the order
+// The f16 parts of the scaled rows 2^wcol[n].x wnk[n] of [N, Kp] in the order
 // the wide kernel's lanes read them: 16-row tile j, 32-k stage ch, part p of
 // `parts`, lane l (row 16 j + l % 16, k 32 ch + 8 (l / 16) .. + 8), 16 bytes
 // each.  Rows past N and k past Kp are zeros.  One part: *rest becomes 1 if
@@ -934,7 +955,7 @@ __global__ __launch_bounds__(256) void weight_exponent_kernel(const float* __res
 // of row n: x the dense ones and, in the high half, those that reach kWBig; y
 // the weights below kTiny that the parts do not hold (column_run).
 __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ wnk,
-                                                            const int* __restrict__ wexp,
+                                                            const int2* __restrict__ wcol,
                                                             u32x4* __restrict__ dst, int N, int Kp,
                                                             int nch, long long pieces, int parts,
                                                             int* __restrict__ rest,
@@ -946,7 +967,7 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restr
   const int ch = static_cast<int>(jc % nch);
   const long long row = (jc / nch) * 16 + (lane & 15);
   const int k0 = ch * KC + 8 * (lane >> 4);
-  const int e = row < N ? wexp[row] : 0;
+  const int e = row < N ? wcol[row].x : 0;
   auto at = [&](int h) {
     return row < N && k0 + h < Kp ? ldexpf(wnk[static_cast<size_t>(row) * Kp + k0 + h], e) : 0.0f;
   };
@@ -1008,29 +1029,29 @@ int split_weights(vk_linear* lin, bool f16_values) {
   // (its smallest values then leave remainders): tried first, and split in two
   // where the kernel finds a remainder.
   for (int parts = f16_values ? 1 : 2; parts <= 2; ++parts) {
-    // one allocation: the parts, the stages' counts, the exponents, the remainder flag
+    // one allocation: the parts, the stages' counts, the columns, the remainder flag
     const size_t bytes = static_cast<size_t>(pieces) * 16 * parts;
     const size_t stat_bytes = (static_cast<size_t>(nch) + 1) * n * sizeof(uint2);
     VK_HIP(hipMalloc(&lin->weight_split,
-                     bytes + stat_bytes + (static_cast<size_t>(n) + 1) * sizeof(int)));
+                     bytes + stat_bytes + (static_cast<size_t>(n) + 1) * sizeof(int2)));
     char* base = static_cast<char*>(lin->weight_split);
     lin->weight_stat = reinterpret_cast<uint2*>(base + bytes);
-    lin->weight_exp = reinterpret_cast<int*>(base + bytes + stat_bytes);
+    lin->weight_col = reinterpret_cast<int2*>(base + bytes + stat_bytes);
     lin->weight_parts = parts;
-    hipLaunchKernelGGL(weight_exponent_kernel, dim3((n + 3) / 4), dim3(256), 0, nullptr,
-                       lin->weight_nk, lin->weight_exp, n, kp);
-    VK_TRY(check_launch("weight_exponent_kernel"));
+    hipLaunchKernelGGL(weight_column_kernel, dim3((n + 3) / 4), dim3(256), 0, nullptr,
+                       lin->weight_nk, lin->weight_col, n, kp);
+    VK_TRY(check_launch("weight_column_kernel"));
     hipLaunchKernelGGL(split_weights_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                       nullptr, lin->weight_nk, lin->weight_exp,
+                       nullptr, lin->weight_nk, lin->weight_col,
                        static_cast<u32x4*>(lin->weight_split), n, kp, static_cast<int>(nch),
-                       pieces, parts, lin->weight_exp + n, lin->weight_stat);
+                       pieces, parts, &lin->weight_col[n].x, lin->weight_stat);
     VK_TRY(check_launch("split_weights_kernel"));
     hipLaunchKernelGGL(stage_totals_kernel, dim3((n + 255) / 256), dim3(256), 0, nullptr,
                        lin->weight_stat, n, static_cast<int>(nch));
     VK_TRY(check_launch("stage_totals_kernel"));
     if (parts == 2) break;
     int rest = 0;
-    VK_HIP(hipMemcpy(&rest, lin->weight_exp + n, sizeof(int), hipMemcpyDeviceToHost));
+    VK_HIP(hipMemcpy(&rest, &lin->weight_col[n].x, sizeof(int), hipMemcpyDeviceToHost));
     if (!rest) return VK_OK;
     VK_HIP(hipFree(lin->weight_split));
     lin->weight_split = nullptr;

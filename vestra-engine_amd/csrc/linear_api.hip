@@ -174,7 +174,7 @@ LinearArgs linear_args(const vk_linear* lin, const vk_tensor* x, size_t rows, vk
   g.x = static_cast<const float*>(x->ptr);
   g.wnk = lin->weight_nk;
   g.wsplit = lin->weight_split;
-  g.wexp = lin->weight_exp;
+  g.wcol = lin->weight_col;
   g.wstat = lin->weight_stat;
   g.wparts = lin->weight_parts;
   g.bias = lin->bias;
@@ -210,7 +210,7 @@ int launch_linear(vk_runtime* rt, const vk_linear* lin, const vk_tensor* x, size
   g.x = static_cast<const float*>(x->ptr);
   g.wnk = lin->weight_nk;
   g.wsplit = lin->weight_split;
-  g.wexp = lin->weight_exp;
+  g.wcol = lin->weight_col;
   g.wstat = lin->weight_stat;
   g.wparts = lin->weight_parts;
   g.bias = lin->bias;
