@@ -70,12 +70,15 @@ constexpr int PITCH = 68;
 constexpr int kSlots = KB * HD / 4;  // float4 of one K (or V) block: 1024
 constexpr float kQScale = 0.125f * 1.44269504088896341f;  // log2(e) / sqrt(64)
 // Scales of the f16 parts (powers of two): K by 2^8, Q (with kQScale) by 2^10,
-// the weights by 2^11 with room for a factor 2^4 above the running max.  |k| of
+// the weights by 2^11 with room for a factor 2^2 above the running max (2^4 saves
+// a few rescales, 0.5% at 12 x 10,392, but leaves more weights where the exponent's
+// argument is rounded at 2^-21: 3.95e-7 of the 64-bit result at 12 x 866 against
+// 3.88e-7; f16 holds 2^4).  |k| of
 // 256 and |q| of 354 no longer fit (queries that meet them run in F32).  A
 // column of V is brought to [2^kVBits, 2 x that) by the largest value of the
 // run's first key block; one of 64 to 128 times that no longer fits.
 constexpr float kKUp = 256.0f, kQUp = 1024.0f, kSDown = 1.0f / 262144.0f;
-constexpr float kPBits = 11.0f, kPDown = 1.0f / 2048.0f, kSlack = 4.0f;
+constexpr float kPBits = 11.0f, kPDown = 1.0f / 2048.0f, kSlack = 2.0f;
 constexpr int kVBits = 9;
 // A query is held whose largest sum (of 64, over scaled V) reaches both: the
 // floors of V (2^-25 of a scaled value) and of the weights (2^-25 each, of
