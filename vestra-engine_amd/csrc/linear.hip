@@ -24,12 +24,14 @@
 // fragment reads from LDS (4 waves: 512 cycles of its 128 bytes a clock)
 // and 16 + 16 KiB from L2; two workgroups a CU cover each other's barriers.  A
 // 128 x 256 tile splits and reads A once for twice the columns: 10,392 x 3072
-// -> 768 in 127 us against 136 (386 TFLOP/s of the product's FLOP, 1,160 of f16
-// MFMA; a large f16 library product reaches 1,243 on the card).  What bounds
-// both is the matrix pipe at the clock that its power allows (about 2.0 GHz,
-// 50% busy); bank conflicts of the staging stores do not show (a conflict-free
-// plane layout measured the same), lines of A touched more often do (a lane
-// per row instead of four: 10-20% slower).
+// -> 768 in 129 us against 138 (380 TFLOP/s of the product's FLOP, 1,140 of f16
+// MFMA; a large f16 library product reaches 1,243 on the card).  No single unit
+// bounds it: at the 2.0 GHz its power allows the matrix pipe is busy 51% of the
+// cycles (38% with GELU and 128 MB of output), waves wait 27-31% of theirs, and
+// the split's VALU work lies between a stage's MFMAs and its barrier.  Bank
+// conflicts of the staging stores do not show (a conflict-free plane layout
+// measured the same), lines of A touched more often do (a lane per row instead
+// of four: 10-20% slower).
 // Grids of few tiles split K over several workgroups per tile (split-K:
 // partial sums in the runtime's work buffer, added in split order by
 // splitk_reduce_kernel).
@@ -49,7 +51,7 @@
 // the code path are those of the separate pass, so the bits are too.
 //
 // Every output is either the split's sum or, where the split may hold its
-// terms less well than F32 does, an F32 one: the wave computes the 16 rows of
+// terms less well than F32 does, an F32 one: the wave computes 64 rows of
 // its columns again with F32 matrix instructions on the f32 operands and takes
 // the outputs in question from there.  Which they are depends on the output's
 // own row and column alone (and the split-K run), so no other row or column of
@@ -1007,13 +1009,19 @@ __global__ __launch_bounds__(256) void stage_totals_kernel(uint2* __restrict__ s
   if (n >= N) return;
   uint2 sum = make_uint2(0, 0);
   stat[n] = sum;
-  for (int ch = 1; ch <= nch; ++ch) {
-    uint2* p = stat + static_cast<size_t>(ch) * N + n;
-    const uint2 v = *p;
-    // the halves of x wrap on their own (read back as differences)
-    sum = make_uint2(((sum.x + v.x) & 0xffffu) | ((sum.x & 0xffff0000u) + (v.x & 0xffff0000u)),
-                     sum.y + v.y);
-    *p = sum;
+  constexpr int kAhead = 16;  // loads in flight (the stores would order them one by one)
+  for (int c0 = 1; c0 <= nch; c0 += kAhead) {
+    uint2 v[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+      v[i] = stat[static_cast<size_t>(c0 + i <= nch ? c0 + i : nch) * N + n];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      // the halves of x wrap on their own (read back as differences)
+      sum = make_uint2(((sum.x + v[i].x) & 0xffffu) | ((sum.x & 0xffff0000u) + (v[i].x & 0xffff0000u)),
+                       sum.y + v[i].y);
+      if (c0 + i <= nch) stat[static_cast<size_t>(c0 + i) * N + n] = sum;
+    }
   }
 }
 
