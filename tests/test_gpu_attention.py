@@ -1,9 +1,9 @@
 """GPU parity of the attention core, `attention_online_f32` (vit_block.rs:363, 559;
 CPU `vestra_kernels::attention`, vit_block.rs:952), through the C ABI.
 
-The GPU computes every score and every probability-weighted sum as an F32
-MFMA dot product and the softmax online (one pass over 64-key blocks), the
-oracle sequentially in f32.  Both are compared with a bound derived from the
+The GPU computes every score and every probability-weighted sum as three f16
+MFMA products of two-part splits (F32 accumulation) and the softmax online (one
+pass over 64-key blocks), the oracle sequentially in f32.  Both are compared with a bound derived from the
 float64 result of the same inputs:
 
   |gpu - oracle| <= 1e-6 + 1e-5*|ref| + E * A + (2*sqrt(n) + nb + 4) * u * B
@@ -66,10 +66,9 @@ def _run(rt, q, k, v, seqs, n):
 @pytest.mark.parametrize("seqs,n", [(1, 1), (3, 37), (2, 64), (2, 65), (1, 129), (12, 866),
                                     (2, 1000), (1, 3000)])
 def test_attention_matches_oracle(rt, rng, seqs, n):
-    """Grids of fewer than two 64-query workgroups per CU split each tile's
-    key blocks over workgroups: 12 x 866 in 3 splits, 2 x 1000 in 8 splits
-    of 2 blocks, 1 x 3000 in 8 splits of 5-6 blocks (ending in the partial
-    block); the others run one workgroup per tile."""
+    """12 x 866 runs in 3 key splits, 2 x 1000 in 8 splits of 2 blocks, 1 x 3000
+    in 8 splits of 5-6 blocks (ending in the partial block); the others run one
+    workgroup per tile (n <= 64: the F32 kernel of one key block)."""
     q, k, v = (normals(rng, seqs, n, 64) for _ in range(3))
     got = _run(rt, q, k, v, seqs, n)
     want = oracle.attention(q, k, v, seqs, n, 64)
@@ -106,10 +105,10 @@ def test_attention_large_scores_and_selection(rt, rng):
 
 @pytest.mark.parametrize("heads,n", [(12, 10392), (16, 3458), (12, 13856), (12, 20784)])
 def test_attention_full_size_sampled_rows(rt, rng, heads, n):
-    """Global layer of the 12-view ViT-B sequence (12 heads over 10,392 rows,
-    each query tile's key blocks in three splits), the ViT-L 1008x672 image
-    (16 heads over 3,458 rows, two splits) and the global layers of 16 and 24
-    views (13,856 and 20,784 rows: five and four splits): every head, 48
+    """Global layer of the 12-view ViT-B sequence (12 heads over 10,392 rows),
+    the ViT-L 1008x672 image (16 heads over 3,458 rows) and the global layers of
+    16 and 24 views (13,856 rows, five key splits, and 20,784), all on eight-wave
+    workgroups, the others unsplit: every head, 48
     sampled query rows (first, last, the special tokens, view boundaries)
     against float64 with the bound above."""
     q, k, v = (normals(rng, heads, n, 64) for _ in range(3))

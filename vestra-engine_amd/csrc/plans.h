@@ -79,9 +79,11 @@ inline int linear_slices_to_provide(long long cus, int M, int N, int K) {
 // read by the sum pass, at about 5.5 TB/s) and the sum pass's launch (about 2
 // us).  The cheapest plan wins; on ties the first shape, then the smaller
 // count.  At least four stages per
-// split; where the shape may split, at most kMaxStages of them (a run's
-// rounding grows with its length: K = 4096, 4.1e-7 of the 64-bit result
-// unsplit, 3.0e-7 in two).  Measured (model's choice; neighbours): 866 x 768 ->
+// split; where the shape may split, at most kMaxStages of them: a run's
+// rounding grows as the root of its length (2.0e-7 of the 64-bit result at 768 k,
+// 3.0e-7 at 2,048, 3.6e-7 at 3,072, 4.1e-7 at 4,096, 5.9e-7 at 8,192), and 96
+// stages keep ViT-B's longest sum in one run and let ViT-L's (K = 4096) take two,
+// which is also the faster there (3,458 rows: 90 us against 97).  Measured (model's choice; neighbours): 866 x 768 ->
 // 2304, 64 x 64 17.2 us (64 x 128 18.2, 128 x 128 29); 866 x 3072 -> 768, 64 x
 // 64 x 3 24.4 (unsplit 35, 64 x 128 x 6 24.3); 1500 x 768 -> 2304, 64 x 128 24.3
 // (64 x 64 27, 128 x 128 30); 3458 x 4096 -> 1024, 128 x 256 x 2 90 (64 x 128
