@@ -98,6 +98,16 @@ def test_queries_that_attend_to_small_rows(rt, rng, s, n, small):
         _assert_close(got[i], q[i], k[i], v[i], f"seq {i}")
 
 
+@pytest.mark.parametrize("s,n", FORMS + [(4, 10392)])
+def test_even_attention_beside_a_few_large_rows(rt, rng, s, n):
+    """Weights all alike and three first keys with V a hundred times the others':
+    outputs far below V's largest values."""
+    q, k, v = (normals(rng, s, n, 64) for _ in range(3))
+    v[:, :3] *= 100
+    v -= v.mean(axis=1, keepdims=True)
+    _check(rt, q * np.float32(0.01), k, v, "even", [0, s - 1])
+
+
 def test_growing_maximum_and_flat_tails(rt, rng):
     """Scores that rise block after block (the running maximum moves each
     time), in steps below the slack, and thousands of weights far below one."""

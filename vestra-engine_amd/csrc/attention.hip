@@ -43,7 +43,7 @@
 // 1,064 us.
 //
 // A query that the split does not hold (a result that is not finite, or one
-// that is small beside V's columns, kHeldMean) is computed again with F32 matrix
+// that is small beside V's columns, kHeldSum) is computed again with F32 matrix
 // instructions by its workgroup, alone: a query's bits depend on its own row and
 // its sequence's K and V only (attention_tile_f32).
 // V of any scale runs at full speed (12 x 866, V x 1e-4: 25 us; judged by one
@@ -80,10 +80,14 @@ constexpr float kQScale = 0.125f * 1.44269504088896341f;  // log2(e) / sqrt(64)
 constexpr float kKUp = 256.0f, kQUp = 1024.0f, kSDown = 1.0f / 262144.0f;
 constexpr float kPBits = 11.0f, kPDown = 1.0f / 2048.0f, kSlack = 2.0f;
 constexpr int kVBits = 9;
-// A query is held whose largest sum (of 64, over scaled V) reaches both: the
-// floors of V (2^-25 of a scaled value) and of the weights (2^-25 each, of
-// random sign) are then below 2^-24 of that sum.
-constexpr float kHeldMean = 0.5f, kHeldSum = 8192.0f;
+// A query is held whose largest sum m (of 64, over scaled V and weights of sum l)
+// has m >= kHeldSum and m^2 >= kHeldSquare l.  The floors are 2^-25 of every scaled
+// value of V and of every weight, of random sign: V's add up to 2^-25 sqrt(sum
+// p^2) <= 2^-25 sqrt(2^13 l), the largest weight being at most 2^13, which the
+// second keeps below 2^-24 m; the weights' to 2^-25 sqrt(n) of V's usual size
+// (2^8), below 2^-24 m for n = 4,096 by the first.  (l / 2 in place of its root took
+// queries again that attend evenly to 10,000 keys beside a few with larger V.)
+constexpr float kHeldSquare = 2048.0f, kHeldSum = 8192.0f;
 constexpr int kFlush = 8;       // blocks between additions to the running total
 constexpr int kRowBytes = 272;  // LDS pitch of 64 values: 2 parts x 128 bytes + 16
 constexpr int kBufBytes = 2 * KB * kRowBytes;  // a block of K and of V
@@ -650,7 +654,7 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
 
   // Which queries did the split hold?  Any value of Q, K or V beyond f16, an
   // infinity or a NaN makes the sums that it enters NaN or infinite; sums that
-  // are all small beside V's columns may show the floors (kHeldMean, kHeldSum).
+  // are all small beside V's columns may show the floors (kHeldSum, kHeldSquare).
   const int qi = q0 + c32;
   const bool mine = live && qi < n;
   {
@@ -672,7 +676,7 @@ __global__ __launch_bounds__(64 * QW, 2) void attention_kernel(const float* __re
     const float m = xor32_pair(most, &other);
     most = fmaxf(m, other);
   }
-  const bool small = !(most >= kHeldMean * l_run && most >= kHeldSum);
+  const bool small = !(most >= kHeldSum && most * most >= kHeldSquare * l_run);
   auto queries = [&](bool x) {  // one bit per query of the wave, from either half
     const uint64_t b = __builtin_amdgcn_ballot_w64(mine && x);
     return static_cast<uint32_t>(b) | static_cast<uint32_t>(b >> 32);
