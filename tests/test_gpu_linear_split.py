@@ -54,7 +54,7 @@ def test_shapes(rt, rng, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(130, 768, 192), (1500, 768, 2304), (10392, 128, 768),
-                                   (10392, 768, 768)])
+                                   (10392, 768, 768), (70, 20, 64), (300, 48, 128)])
 @pytest.mark.parametrize("xs,ws", [(1e-6, 1.0), (1e-3, 1e-20), (1e5, 1e-3), (1e25, 1e-30),
                                    (1e-30, 1e10), (3e4, 1.0), (1e-38, 1.0)])
 def test_value_ranges(rt, rng, m, k, n, xs, ws):
@@ -147,7 +147,8 @@ def test_mixed_sizes_within_a_row_and_a_column(rt, rng, m, k, n, small):
         _check(got[::2, ::2], x[::2], w[:, ::2], b[::2], f"column, met alone, {large} large")
 
 
-@pytest.mark.parametrize("m,k", [(130, 192), (1500, 768), (10392, 128), (4100, 1024)])
+@pytest.mark.parametrize("m,k", [(130, 192), (1500, 768), (10392, 128), (4100, 1024), (70, 16),
+                                 (300, 48)])
 def test_selecting_weights_copy(rt, rng, m, k):
     """A column with a single weight of 1 returns its channel's bits; a row with
     a single 1 the weights of that channel."""

@@ -71,7 +71,8 @@
 //    whose weight is at least 8.  Taken again unless one of the two reaches
 //    `need`: the floor then stays below 2^-24 s;
 //  * a sum of few terms, which F32 adds with next to no rounding (a one-hot
-//    column copies): fewer than 8 groups of the row reach 1, or of the column 8.
+//    column copies): fewer than a quarter of the run's groups, 8 at most, reach 1
+//    in the row, or 8 in the column.
 // Ordinary rows (layer-normalised, GELU outputs, attention outputs) and dense
 // columns pass as a whole; then an output costs only the test that it is finite.
 // The scale and the counts take 0.5 to 1.1 us of a launch of one image (866 x 768
@@ -105,9 +106,11 @@ constexpr float kTiny = 1.0f / 8192.0f, kXBig = 1.0f, kWBig = 8.0f;
 // A row's typical value is brought to [2^kRowBits, 2 x that), its largest one
 // (of those looked at) below 2^(kRowMaxBits + 1).
 constexpr int kRowBits = 6, kRowMaxBits = 9;
-constexpr int kFewGroups = 8;      // sums of fewer groups than this are F32 sums
-// The linears of the split: at least kFewGroups groups, counts of 16 bits.
-constexpr int kMinSplitK = 8 * kFewGroups, kMaxSplitK = 1 << 18;
+// Sums of fewer groups than this are F32 sums: a quarter of the run's, 2 to 8.
+__device__ __forceinline__ int few_groups(int groups) {
+  return groups >= 32 ? 8 : (groups >= 8 ? groups / 4 : 2);
+}
+constexpr int kMaxSplitK = 1 << 18;  // counts of 16 bits; longer sums are F32 sums
 constexpr int kZeroColumn = 1 << 20;  // exponent of a column of zeros
 constexpr int kZeroRowExp = 126;      // and of a row without a value in the sample
 constexpr int kRowBytes = 144;     // LDS pitch of a row of A: 2 parts x 64 bytes + 16
@@ -430,8 +433,9 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
   // of the one after.  A buffer is written again in the stage after the one
   // that read it, with a barrier in between.
   u32x4 b0[KS][NU][NP], b1[KS][NU][NP];
-  const bool split_k = g.K >= kMinSplitK && g.K < kMaxSplitK;  // else F32 throughout
-  const int groups = 4 * (c_end - c_begin);
+  const bool split_k = g.K < kMaxSplitK;  // else F32 throughout
+  const int k_end = c_end * KC < g.K ? c_end * KC : g.K;
+  const int groups = (k_end - c_begin * KC + 7) / 8, few = few_groups(groups);
   auto col_of = [&](int u) { return n0 + wave * WN + u * 16 + (lane & 15); };
   int cexp[NU];
   float cfloor[NU];
@@ -509,7 +513,7 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
     for (int u = 0; u < NU; ++u) {
       cr[u] = column_run(cr0[u], cr1[u]);
       look |= (cexp[u] != kZeroColumn) &
-              ((cr[u].any < kFewGroups) |
+              ((cr[u].any < few) |
                (8 * (cr[u].dense - groups) - 16 * cr[u].tiny < -6 * groups));
     }
 #pragma unroll
@@ -525,12 +529,12 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
     bool plain_rows = true;
 #pragma unroll
     for (int i = 0; i < kVR; ++i) {
-      // a stage past the run's end counted one piece of zeros
-      const int tiny = static_cast<int>(
-          quad_sum(rtiny[i] - ((c_end - c_begin) % KS != 0 ? 1u : 0u)));
+      // pieces past the run's end were zeros and counted
+      const int past = 4 * KS * ((c_end - c_begin + KS - 1) / KS) - groups;
+      const int tiny = static_cast<int>(quad_sum(rtiny[i])) - past;
       const int big = static_cast<int>(quad_sum(rbig[i]));
       const int e = static_cast<int>(__float_as_uint(rscale[i]) >> 23) - 127;
-      plain_rows &= e == kZeroRowExp || (big >= kFewGroups && 8 * big - 4 * tiny >= 6 * groups);
+      plain_rows &= e == kZeroRowExp || (big >= few && 8 * big - 4 * tiny >= 6 * groups);
       if (piece == 0) {
         row_exp[slot_row(i)] = e;
         row_cnt[slot_row(i)] = tiny << 16 | big;
@@ -588,7 +592,7 @@ __global__ __launch_bounds__(64 * waves_for(TN), 2) void linear_wide_kernel(Line
                                static_cast<float>(16 * cr[u].tiny);
             const bool held =
                 e[r] == kZeroRowExp || cexp[u] == kZeroColumn ||
-                (big >= kFewGroups && cr[u].any >= kFewGroups &&
+                (big >= few && cr[u].any >= few &&
                  fmaxf(static_cast<float>(8 * (big + cr[u].dense - groups)), fabsf(v)) >= need);
             if (!held || !vks::is_finite(v)) again[i] |= 1u << (4 * u + r);
             acc[t][u][r] = __builtin_amdgcn_ldexpf(v, -e[r] - cexp[u]);
